@@ -23,7 +23,7 @@ LIB = os.path.join(LIBDIR, "libcucim_amd.so")
 OBJ = os.path.join(ROOT, "_build")
 
 SOURCES = ["hc_host.hip", "k_correlate.hip", "k_hessian.hip", "k_pointwise.hip",
-           "k_stencil2d.hip", "k_ridges.hip", "k_cnn3d.hip",
+           "k_stencil2d.hip", "k_ridges.hip", "k_cnn3d.hip", "k_cnn3d_bwd.hip",
            "k_frangi_check.hip", "k_eig_nd.hip", "k_measure.hip",
            "hc_taps.hip", "hc_wsi.hip"]
 

@@ -93,6 +93,10 @@ ENTRY_POINTS = (
     "hc_cnn3d_dgrad",
     "hc_cnn3d_wgrad",
     "hc_cnn3d_mse_grad",
+    "hc_cnn3d_mse_grad_batch",
+    "hc_cnn3d_wgrad_work",
+    "hc_cnn3d_wgrad_batch",
+    "hc_cnn3d_dgrad_batch",
     "hc_cnn3d_adam",
     "hc_frangi_check",
 )
@@ -195,6 +199,11 @@ _SIGNATURES = {
     "hc_cnn3d_dgrad": ([_v, _v, _v, _i, _i, _i, _i, _i, _v], _i),
     "hc_cnn3d_wgrad": ([_v, _v, _v, _v, _i, _i, _i, _i, _i, _v], _i),
     "hc_cnn3d_mse_grad": ([_v, _v, _v, ctypes.c_int64, _v, _v], _i),
+    "hc_cnn3d_mse_grad_batch": ([_v, _v, _v, ctypes.c_int64, ctypes.c_int64, _v, _v], _i),
+    "hc_cnn3d_wgrad_work": ([_i, _i], ctypes.c_int64),
+    "hc_cnn3d_wgrad_batch": ([_v, _v, _v, _v, ctypes.c_int64, _i, _i, _i, _i, _i, _v,
+                              ctypes.c_int64, _v], _i),
+    "hc_cnn3d_dgrad_batch": ([_v, _v, _v, _v, ctypes.c_int64, _i, _i, _i, _i, _i, _v], _i),
     "hc_cnn3d_adam": ([_v, _v, _v, _v, ctypes.c_int64, _d, _d, _d, _d, _i, _v], _i),
     "hc_frangi_check": ([_A, _A, _v, _i, _v, _v, _P(ctypes.c_int32), _i, _i, _d, _d, _d, _v,
                          _v, _v], _i),

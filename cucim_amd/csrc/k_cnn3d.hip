@@ -28,34 +28,12 @@
 #include <cmath>
 #include <cstring>
 
-#include "hc_common.h"
+#include "hc_cnn.h"
 
 namespace hc {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
 constexpr int kBY = 8, kBX = 16;        // output block rows / columns
 constexpr int kTY = kBY + 2, kTX = kBX + 2;  // input tile rows / columns
-
-__device__ __forceinline__ float bf2f(__bf16 v) { return (float)v; }
-__device__ __forceinline__ __bf16 f2bf(float v) { return (__bf16)v; }  // RNE
-
-// GELU in its tanh form (torch.nn.GELU(approximate="tanh")):
-// 0.5 x (1 + tanh(z / 2)) = x * sigmoid(z), z = 2 sqrt(2/pi) (x + 0.044715 x^3),
-// with the hardware exp and reciprocal (the network is trained with this
-// same function and its derivative).
-__device__ __forceinline__ float gelu_z(float x) {
-  return 1.5957691216057308f * fmaf(0.044715f * x, x * x, x);
-}
-__device__ __forceinline__ float gelu(float x) {
-  return x * __builtin_amdgcn_rcpf(1.0f + __expf(-gelu_z(x)));
-}
-__device__ __forceinline__ float gelu_grad(float x) {
-  const float s = __builtin_amdgcn_rcpf(1.0f + __expf(-gelu_z(x)));
-  const float dz = 1.5957691216057308f * fmaf(3.0f * 0.044715f, x * x, 1.0f);
-  return fmaf(x * s * (1.0f - s), dz, s);
-}
 
 enum { ACT_NONE = 0, ACT_GELU = 1, ACT_CLAMP01 = 2 };
 
@@ -66,8 +44,8 @@ struct ConvArgs {
   const bf16x8* wpk;  // packed weights: [chunk][ntile][64 lanes]
   const float* bias;  // CO
   int D, H, W;        // input extents
-  int nbx, nby;       // blocks along x, y
-  int64_t nblocks;
+  int nbx, nby, nbz;  // blocks along x, y, z of one patch
+  int64_t nblocks;    // of the whole batch
 };
 
 template <int CI>
@@ -76,13 +54,19 @@ struct ConvGeom {
   static constexpr int NCH = (K + 31) / 32;  // K chunks of 32
 };
 
-// Block b of the output grid (x fastest) -> origin.
+// Block b of the output grid (x fastest, patches slowest; fewer than 2^31
+// blocks) -> origin; returns the patch.
 template <int BZ>
-__device__ __forceinline__ void block_origin(const ConvArgs& a, int64_t b, int& x0, int& y0,
-                                             int& z0) {
-  x0 = (int)(b % a.nbx) * kBX;
-  y0 = (int)((b / a.nbx) % a.nby) * kBY;
-  z0 = (int)(b / ((int64_t)a.nbx * a.nby)) * BZ;
+__device__ __forceinline__ int64_t block_origin(const ConvArgs& a, int64_t b, int& x0, int& y0,
+                                                int& z0) {
+  unsigned q = (unsigned)b;
+  unsigned r = q / (unsigned)a.nbx;
+  x0 = (int)(q - r * a.nbx) * kBX;
+  q = r / (unsigned)a.nby;
+  y0 = (int)(r - q * a.nby) * kBY;
+  r = q / (unsigned)a.nbz;
+  z0 = (int)(q - r * a.nbz) * BZ;
+  return r;
 }
 
 // BZ output planes per block, two waves per plane (4 rows of 16 voxels each).
@@ -108,7 +92,7 @@ __global__ __launch_bounds__(128 * BZ) void k_conv3d_mfma(const ConvArgs a) {
   // input tile of block b: global -> registers (VEC) or straight to LDS
   auto fetch = [&](int64_t b, bf16x8 (&r)[NPF]) {
     int x0, y0, z0;
-    block_origin<BZ>(a, b, x0, y0, z0);
+    const int64_t n = block_origin<BZ>(a, b, x0, y0, z0);
 #pragma unroll
     for (int u = 0; u < NPF; ++u) {
       const int e = tid + NTH * u;
@@ -120,7 +104,7 @@ __global__ __launch_bounds__(128 * BZ) void k_conv3d_mfma(const ConvArgs a) {
         const int gx = x0 + tx, gy = y0 + ty, gz = z0 + tz;
         if (gx < a.W && gy < a.H && gz < a.D)
           val = reinterpret_cast<const bf16x8*>(
-              a.in + (((int64_t)gz * a.H + gy) * a.W + gx) * CI)[v];
+              a.in + (((n * a.D + gz) * a.H + gy) * a.W + gx) * CI)[v];
       }
       r[u] = val;
     }
@@ -134,14 +118,14 @@ __global__ __launch_bounds__(128 * BZ) void k_conv3d_mfma(const ConvArgs a) {
   };
   auto stage_scalar = [&](int64_t b) {
     int x0, y0, z0;
-    block_origin<BZ>(a, b, x0, y0, z0);
+    const int64_t n = block_origin<BZ>(a, b, x0, y0, z0);
     for (int e = tid; e < TILE; e += NTH) {
       const int c = e % CI, vox = e / CI;
       const int tx = vox % kTX, ty = (vox / kTX) % kTY, tz = vox / (kTX * kTY);
       const int gx = x0 + tx, gy = y0 + ty, gz = z0 + tz;
       __bf16 val = (__bf16)0.0f;
       if (gx < a.W && gy < a.H && gz < a.D)
-        val = a.in[(((int64_t)gz * a.H + gy) * a.W + gx) * CI + c];
+        val = a.in[(((n * a.D + gz) * a.H + gy) * a.W + gx) * CI + c];
       T[e] = val;
     }
   };
@@ -154,7 +138,7 @@ __global__ __launch_bounds__(128 * BZ) void k_conv3d_mfma(const ConvArgs a) {
     const int64_t blk = base + slot;
     if (blk >= a.nblocks) break;  // uniform per work-group
     int x0, y0, z0;
-    block_origin<BZ>(a, blk, x0, y0, z0);
+    const int64_t pn = block_origin<BZ>(a, blk, x0, y0, z0);
     __syncthreads();  // the previous block is done with T
     if (VEC) {
       put(pf);
@@ -239,7 +223,7 @@ __global__ __launch_bounds__(128 * BZ) void k_conv3d_mfma(const ConvArgs a) {
           float y = p;
           if (ACT == ACT_GELU) y = gelu(p);
           if (ACT == ACT_CLAMP01) y = fminf(fmaxf(p, 0.f), 1.f);
-          const int64_t o = (((int64_t)gz * OH + gy) * OW + gx) * CO + co;
+          const int64_t o = (((pn * OD + gz) * OH + gy) * OW + gx) * CO + co;
           if (inside && a.pre) a.pre[o] = p;
           if (STAGE_OUT) {
             O[((oz * kBY + oy0 + m) * kBX + lx) * CO + co] = f2bf(y);
@@ -261,7 +245,7 @@ __global__ __launch_bounds__(128 * BZ) void k_conv3d_mfma(const ConvArgs a) {
         const int gx = x0 + lx, gy = y0 + ly, gzz = z0 + lz;
         if (gx < OW && gy < OH && gzz < OD)
           reinterpret_cast<bf16x8*>(reinterpret_cast<__bf16*>(a.out) +
-                                    (((int64_t)gzz * OH + gy) * OW + gx) * CO)[v] =
+                                    (((pn * OD + gzz) * OH + gy) * OW + gx) * CO)[v] =
               reinterpret_cast<const bf16x8*>(O)[e];
       }
     }
@@ -427,12 +411,12 @@ namespace {
 int64_t grid_of(int64_t n) { return n <= 0 ? 1 : std::min<int64_t>((n + 255) / 256, 256 * 64); }
 
 template <int CI, int CO, int ACT, bool F32, int BZ>
-int conv_launch(ConvArgs a, hipStream_t st) {
+int conv_launch(ConvArgs a, int64_t batch, hipStream_t st) {
   constexpr int NCH = ConvGeom<CI>::NCH, NT = (CO + 15) / 16;
   a.nbx = (a.W - 2 + kBX - 1) / kBX;
   a.nby = (a.H - 2 + kBY - 1) / kBY;
-  const int nbz = (a.D - 2 + BZ - 1) / BZ;
-  a.nblocks = (int64_t)a.nbx * a.nby * nbz;
+  a.nbz = (a.D - 2 + BZ - 1) / BZ;
+  a.nblocks = batch * a.nbx * a.nby * a.nbz;
   if (a.nblocks > 0x7fffffff) return fail(HC_ERR_VALUE, "volume too large");
   // weights, then the input tile (also the output block's staging area)
   const size_t tile =
@@ -478,12 +462,16 @@ int hc_cnn3d_pack(const float* w_dev, void* packed_dev, int ci, int co, void* st
 int hc_cnn3d_conv(const hc_array* in, const hc_array* out, const void* packed,
                   const float* bias_dev, int act, float* pre_dev, void* stream) {
   if (!in || !out || !packed || !bias_dev) return fail(HC_ERR_VALUE, "null argument");
-  if (in->dtype != HC_BFLOAT16 || in->ndim != 4 || !is_c_contiguous(in))
-    return fail(HC_ERR_VALUE, "input must be a C-contiguous (D, H, W, C) bfloat16 array");
-  if (out->ndim != 4 || !is_c_contiguous(out))
-    return fail(HC_ERR_VALUE, "output must be a C-contiguous (D-2, H-2, W-2, C) array");
-  const int ci = (int)in->shape[3], co = (int)out->shape[3];
-  for (int d = 0; d < 3; ++d)
+  if (in->dtype != HC_BFLOAT16 || (in->ndim != 4 && in->ndim != 5) || !is_c_contiguous(in))
+    return fail(HC_ERR_VALUE, "input must be a C-contiguous ([B,] D, H, W, C) bfloat16 array");
+  if (out->ndim != in->ndim || !is_c_contiguous(out))
+    return fail(HC_ERR_VALUE, "output must be a C-contiguous ([B,] D-2, H-2, W-2, C) array");
+  const int d0 = in->ndim - 4;  // a leading batch dimension
+  const int64_t batch = d0 ? in->shape[0] : 1;
+  if (d0 && out->shape[0] != batch) return fail(HC_ERR_VALUE, "batch sizes differ");
+  if (batch == 0) return HC_OK;
+  const int ci = (int)in->shape[d0 + 3], co = (int)out->shape[d0 + 3];
+  for (int d = d0; d < d0 + 3; ++d)
     if (out->shape[d] != in->shape[d] - 2 || in->shape[d] < 3)
       return fail(HC_ERR_VALUE, "valid convolution: output extents are input extents - 2");
   if (((uintptr_t)in->data | (uintptr_t)packed) % 16)
@@ -495,20 +483,20 @@ int hc_cnn3d_conv(const hc_array* in, const hc_array* out, const void* packed,
   a.pre = pre_dev;
   a.wpk = (const bf16x8*)packed;
   a.bias = bias_dev;
-  a.D = (int)in->shape[0];
-  a.H = (int)in->shape[1];
-  a.W = (int)in->shape[2];
+  a.D = (int)in->shape[d0];
+  a.H = (int)in->shape[d0 + 1];
+  a.W = (int)in->shape[d0 + 2];
   hipStream_t st = (hipStream_t)stream;
   const bool f32 = out->dtype == HC_FLOAT32;
   if (!f32 && out->dtype != HC_BFLOAT16) return fail(HC_ERR_VALUE, "output must be bf16 or f32");
   if (ci == 1 && co == 24 && act == ACT_GELU && !f32)
-    return conv_launch<1, 24, ACT_GELU, false, 2>(a, st);
+    return conv_launch<1, 24, ACT_GELU, false, 2>(a, batch, st);
   if (ci == 24 && co == 24 && act == ACT_GELU && !f32)
-    return conv_launch<24, 24, ACT_GELU, false, 4>(a, st);
+    return conv_launch<24, 24, ACT_GELU, false, 4>(a, batch, st);
   if (ci == 24 && co == 1 && act == ACT_CLAMP01 && f32)
-    return conv_launch<24, 1, ACT_CLAMP01, true, 4>(a, st);
+    return conv_launch<24, 1, ACT_CLAMP01, true, 4>(a, batch, st);
   if (ci == 24 && co == 1 && act == ACT_NONE && f32)
-    return conv_launch<24, 1, ACT_NONE, true, 4>(a, st);
+    return conv_launch<24, 1, ACT_NONE, true, 4>(a, batch, st);
   return fail(HC_ERR_UNSUPPORTED, "layer shape / activation not compiled");
 }
 
@@ -564,13 +552,20 @@ int hc_cnn3d_wgrad(const void* x_bf16, const float* dy, float* dw, float* db, in
   return HC_OK;
 }
 
+int hc_cnn3d_mse_grad_batch(const float* y, const float* t, float* g, int64_t n, int64_t batch,
+                            float* loss, void* stream) {
+  if (!y || !t || !g || !loss || n <= 0 || batch <= 0) return fail(HC_ERR_VALUE, "bad argument");
+  hipStream_t st = (hipStream_t)stream;
+  const int64_t total = n * batch;
+  HC_LAUNCH("k_mse_grad", st, k_mse_grad,
+            dim3((unsigned)std::min<int64_t>(grid_of(total), 1024)), dim3(256), 0, y, t, g, total,
+            1.0f / (float)n, loss);
+  return HC_OK;
+}
+
 int hc_cnn3d_mse_grad(const float* y, const float* t, float* g, int64_t n, float* loss,
                       void* stream) {
-  if (!y || !t || !g || !loss || n <= 0) return fail(HC_ERR_VALUE, "bad argument");
-  hipStream_t st = (hipStream_t)stream;
-  HC_LAUNCH("k_mse_grad", st, k_mse_grad, dim3((unsigned)std::min<int64_t>(grid_of(n), 1024)),
-            dim3(256), 0, y, t, g, n, 1.0f / (float)n, loss);
-  return HC_OK;
+  return hc_cnn3d_mse_grad_batch(y, t, g, n, 1, loss, stream);
 }
 
 int hc_cnn3d_adam(float* p, const float* g, float* m, float* v, int64_t n, double lr,

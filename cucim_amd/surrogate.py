@@ -105,23 +105,25 @@ class FrangiSurrogate:
         return out
 
     def forward(self, x, keep=False, final_act=2, bufs=None, out=None):
-        """x: (D, H, W, 1) bf16 -> (D-10, H-10, W-10) float32.  keep: return
-        the per-layer inputs and pre-activations (training)."""
+        """x: ([B,] D, H, W, 1) bf16 -> ([B,] D-10, H-10, W-10) float32.  keep:
+        return the per-layer inputs and pre-activations (training)."""
         lib = _lib.lib()
         acts, pres = [x], []
         cur = x
+        lead = tuple(int(s) for s in x.shape[:-4])
         for i, (ci, co, act) in enumerate(LAYERS):
-            D, H, W = (int(s) - 2 for s in cur.shape[:3])
+            D, H, W = (int(s) - 2 for s in cur.shape[-4:-1])
+            shape = lead + (D, H, W, co)
             last = i == len(LAYERS) - 1
             if last:
-                dst = out.view(D, H, W, 1) if out is not None else \
-                    torch.empty((D, H, W, 1), dtype=torch.float32, device=_dev())
+                dst = out.view(shape) if out is not None else \
+                    torch.empty(shape, dtype=torch.float32, device=_dev())
                 act = final_act
             elif bufs is not None:
-                dst = bufs[i % 2][: D * H * W * co].view(D, H, W, co)
+                dst = bufs[i % 2][: math.prod(shape)].view(shape)
             else:
-                dst = torch.empty((D, H, W, co), dtype=torch.bfloat16, device=_dev())
-            pre = torch.empty((D, H, W, co), dtype=torch.float32, device=_dev()) if keep else None
+                dst = torch.empty(shape, dtype=torch.bfloat16, device=_dev())
+            pre = torch.empty(shape, dtype=torch.float32, device=_dev()) if keep else None
             _check(lib.hc_cnn3d_conv(_array.hc_array(cur), _array.hc_array(dst),
                                      self.packed[i].data_ptr(), self.b[i].data_ptr(), act,
                                      None if pre is None else pre.data_ptr(),
@@ -130,7 +132,7 @@ class FrangiSurrogate:
                 pres.append(pre)
                 acts.append(dst)
             cur = dst
-        y = cur.view(cur.shape[:3])
+        y = cur.view(cur.shape[:-1])
         return (y, acts, pres) if keep else y
 
     def __call__(self, vol, mode="reflect", cval=0.0):
@@ -170,6 +172,33 @@ class FrangiSurrogate:
             self._step = 0
         return self._gw, self._gb
 
+    def _backward(self, x, t, gw, gb, loss):
+        """Forward and backward of a batch (B, D, H, W, 1) with targets
+        (B, D-10, H-10, W-10): one launch per layer and direction over all
+        its patches; adds to the gradients and the loss."""
+        lib = _lib.lib()
+        st = _array.stream()
+        B = int(x.shape[0])
+        y, acts, pres = self.forward(x, keep=True, final_act=0)
+        g = torch.empty_like(y)
+        _check(lib.hc_cnn3d_mse_grad_batch(y.data_ptr(), t.data_ptr(), g.data_ptr(),
+                                           y.numel() // B, B, loss.data_ptr(), st), "mse")
+        for i in range(len(LAYERS) - 1, -1, -1):
+            ci, co, _ = LAYERS[i]
+            D, H, W = (int(s) for s in acts[i].shape[1:4])
+            n = lib.hc_cnn3d_wgrad_work(ci, co)
+            work = torch.empty(n, dtype=torch.float32, device=_dev())
+            _check(lib.hc_cnn3d_wgrad_batch(acts[i].data_ptr(), g.data_ptr(), gw[i].data_ptr(),
+                                            gb[i].data_ptr(), B, D, H, W, ci, co,
+                                            work.data_ptr(), n, st), "wgrad")
+            if i > 0:
+                # the gradient of the layer before's pre-activations
+                dx = torch.empty((B, D, H, W, ci), dtype=torch.float32, device=_dev())
+                _check(lib.hc_cnn3d_dgrad_batch(g.data_ptr(), self.w[i].data_ptr(),
+                                                pres[i - 1].data_ptr(), dx.data_ptr(), B, D, H,
+                                                W, ci, co, st), "dgrad")
+                g = dx
+
     def train_step(self, xs, ts, lr=1e-3):
         """One Adam step on a batch: xs list of (64, 64, 64, 1) bf16 inputs,
         ts list of (54, 54, 54) float32 targets.  Returns the mean loss
@@ -180,26 +209,8 @@ class FrangiSurrogate:
         for g in gw + gb:
             g.zero_()
         loss = torch.zeros(1, dtype=torch.float32, device=_dev())
-        for x, t in zip(xs, ts):
-            y, acts, pres = self.forward(x, keep=True, final_act=0)
-            g = torch.empty_like(y)
-            _check(lib.hc_cnn3d_mse_grad(y.data_ptr(), t.data_ptr(), g.data_ptr(), y.numel(),
-                                         loss.data_ptr(), st), "mse")
-            g = g.view(*y.shape, 1)
-            for i in range(len(LAYERS) - 1, -1, -1):
-                ci, co, act = LAYERS[i]
-                xin = acts[i]
-                D, H, W = (int(s) for s in xin.shape[:3])
-                if act == 1:
-                    _check(lib.hc_cnn3d_gelu_bwd(g.data_ptr(), pres[i].data_ptr(), g.numel(),
-                                                 st), "gelu bwd")
-                _check(lib.hc_cnn3d_wgrad(xin.data_ptr(), g.data_ptr(), gw[i].data_ptr(),
-                                          gb[i].data_ptr(), D, H, W, ci, co, st), "wgrad")
-                if i > 0:
-                    dx = torch.empty((D, H, W, ci), dtype=torch.float32, device=_dev())
-                    _check(lib.hc_cnn3d_dgrad(g.data_ptr(), self.w[i].data_ptr(),
-                                              dx.data_ptr(), D, H, W, ci, co, st), "dgrad")
-                    g = dx
+        for x, t in _batches(xs, ts):
+            self._backward(x, t, gw, gb, loss)
         self._step += 1
         inv = 1.0 / len(xs)
         for i in range(len(LAYERS)):
@@ -211,6 +222,37 @@ class FrangiSurrogate:
                                          self._step, st), "adam")
         self.repack()
         return loss * inv
+
+
+# Input voxels of one training batch: eight 64^3 patches (their activations
+# and pre-activations take 1.2 GB).
+_BATCH_VOXELS = 8 * 64 ** 3
+
+
+def _batches(xs, ts):
+    """Consecutive patches of one shape stacked along a new first dimension,
+    at most _BATCH_VOXELS input voxels (at least one patch) each.  A patch
+    whose input or target is not a dense array of the expected shape goes
+    alone."""
+    def shape_of(x, t):
+        ok = (x.dim() == 4 and x.is_contiguous() and t.dtype == torch.float32
+              and tuple(t.shape) == tuple(s - 2 * HALO for s in x.shape[:3]))
+        return (tuple(x.shape), x.dtype, x.device, t.device) if ok else None
+
+    pairs = list(zip(xs, ts))
+    i = 0
+    while i < len(pairs):
+        shape = shape_of(*pairs[i])
+        most = 1 if shape is None else max(1, _BATCH_VOXELS // pairs[i][0].numel())
+        j = i + 1
+        while j < len(pairs) and j - i < most and shape_of(*pairs[j]) == shape:
+            j += 1
+        if j - i == 1:
+            yield pairs[i][0][None], pairs[i][1][None]
+        else:
+            yield (torch.stack([p[0] for p in pairs[i:j]]),
+                   torch.stack([p[1] for p in pairs[i:j]]))
+        i = j
 
 
 # ------------------------------------------------------------------ data --

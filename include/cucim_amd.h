@@ -266,8 +266,9 @@ int hc_cnn3d_packed_size(int ci, int co);
 int hc_cnn3d_pack(const float* w_dev, void* packed_dev, int ci, int co, void* stream);
 /* out (D-2, H-2, W-2, co) = act(conv(in (D, H, W, ci)) + bias); out bfloat16,
  * or float32 for the single-channel last layer; pre_dev (float32, out's
- * shape) receives the pre-activation when not NULL (training).  Compiled
- * layer shapes: 1->24 GELU, 24->24 GELU, 24->1 none / clamp. */
+ * shape) receives the pre-activation when not NULL (training).  Both arrays
+ * may have a leading batch dimension.  Compiled layer shapes: 1->24 GELU,
+ * 24->24 GELU, 24->1 none / clamp. */
 int hc_cnn3d_conv(const hc_array* in, const hc_array* out, const void* packed,
                   const float* bias_dev, int act, float* pre_dev, void* stream);
 /* out (D+2p, H+2p, W+2p[, 1]) bfloat16 = boundary-extended float32 in */
@@ -281,6 +282,19 @@ int hc_cnn3d_dgrad(const float* dy, const float* w, float* dx, int D, int H, int
                    int co, void* stream);
 int hc_cnn3d_wgrad(const void* x_bf16, const float* dy, float* dw, float* db, int D, int H,
                    int W, int ci, int co, void* stream);
+/* the same over a batch of equally sized patches, for the compiled layer
+ * shapes (1->24, 24->24, 24->1; no input gradient for 1->24): matrix-core
+ * kernels.  work: hc_cnn3d_wgrad_work(ci, co) floats; pre (dx's shape, may be
+ * NULL): dx is also multiplied by gelu'(pre); n: elements of one patch.
+ * Arrays 16-byte aligned. */
+int64_t hc_cnn3d_wgrad_work(int ci, int co);
+int hc_cnn3d_wgrad_batch(const void* x_bf16, const float* dy, float* dw, float* db, int64_t batch,
+                         int D, int H, int W, int ci, int co, float* work, int64_t work_elems,
+                         void* stream);
+int hc_cnn3d_dgrad_batch(const float* dy, const float* w, const float* pre, float* dx,
+                         int64_t batch, int D, int H, int W, int ci, int co, void* stream);
+int hc_cnn3d_mse_grad_batch(const float* y, const float* t, float* g, int64_t n, int64_t batch,
+                            float* loss, void* stream);
 int hc_cnn3d_mse_grad(const float* y, const float* t, float* g, int64_t n, float* loss,
                       void* stream);
 int hc_cnn3d_adam(float* p, const float* g, float* m, float* v, int64_t n, double lr,

@@ -1,0 +1,117 @@
+"""The matrix-core weight and input gradients over batches of patches against
+float64 autograd, and a training step over stacked patches against the same
+step patch by patch.
+
+A float32 sum of n products differs from the exact one by at most
+n 2^-24 sum |products| (one rounding of half an ulp per addition, the products
+of the matrix core being exact or rounded once), which bounds every element
+here; the 512 partial sums add at most 512 more roundings."""
+
+import numpy as np
+import pytest
+import torch
+import torch.nn.functional as Fnn
+
+pytestmark = pytest.mark.gpu
+
+EPS = 2.0 ** -24
+
+
+def _conv(x, w, b=None):
+    """x: (B, D, H, W, ci), w: (27, ci, co), float64."""
+    ci, co = w.shape[1:]
+    k = w.view(3, 3, 3, ci, co).permute(4, 3, 0, 1, 2)
+    return Fnn.conv3d(x.permute(0, 4, 1, 2, 3), k, b).permute(0, 2, 3, 4, 1)
+
+
+def _grads(x, w, dy):
+    x, w = x.clone().requires_grad_(True), w.clone().requires_grad_(True)
+    b = torch.zeros(w.shape[2], dtype=torch.float64, requires_grad=True)
+    _conv(x, w, b).backward(dy)
+    return x.grad, w.grad, b.grad
+
+
+@pytest.mark.parametrize("ci,co", [(24, 24), (1, 24), (24, 1)])
+@pytest.mark.parametrize("shape", [(1, 3, 3, 3), (2, 4, 10, 18), (3, 5, 11, 19), (1, 20, 3, 35),
+                                   (2, 13, 27, 9)])
+def test_batched_gradients(gpu, ci, co, shape):
+    from cucim_amd import _array
+    from cucim_amd import _lib as L
+
+    lib, st = L.lib(), _array.stream()
+    g = torch.Generator().manual_seed(sum(shape) * 31 + ci)
+    B, D, H, W = shape
+    x = torch.randn(shape + (ci,), generator=g).to(torch.bfloat16)
+    w = torch.randn((27, ci, co), generator=g) / 25
+    dy = torch.randn((B, D - 2, H - 2, W - 2, co), generator=g)
+    ref = _grads(x.double(), w.double(), dy.double())
+    mag = _grads(x.double().abs(), w.double().abs(), dy.double().abs())
+    xd, wd, dyd = x.cuda(), w.cuda(), dy.cuda()
+    n = lib.hc_cnn3d_wgrad_work(ci, co)
+    work = torch.full((n,), float("nan"), device="cuda")
+    dw, db = torch.ones((27, ci, co), device="cuda"), torch.ones(co, device="cuda")
+    L.check(lib.hc_cnn3d_wgrad_batch(xd.data_ptr(), dyd.data_ptr(), dw.data_ptr(), db.data_ptr(),
+                                     B, D, H, W, ci, co, work.data_ptr(), n, st))
+    terms = B * (D - 2) * (H - 2) * (W - 2) + 512 + 1
+    for got, r, m in ((dw, ref[1], mag[1]), (db, ref[2], mag[2])):
+        err = (got.double().cpu() - 1 - r).abs()  # both accumulate (here: onto ones)
+        assert bool((err <= terms * EPS * (m + 1)).all())
+    if ci == 1:
+        rc = lib.hc_cnn3d_dgrad_batch(dyd.data_ptr(), wd.data_ptr(), None, xd.data_ptr(), B, D, H,
+                                      W, ci, co, st)
+        assert rc == L.ERR_UNSUPPORTED
+        return
+    pre = torch.randn(shape + (ci,), generator=g)
+    for p in (None, pre):
+        dx = torch.full(shape + (ci,), float("nan"), device="cuda")
+        pd = None if p is None else p.cuda()
+        L.check(lib.hc_cnn3d_dgrad_batch(dyd.data_ptr(), wd.data_ptr(),
+                                         None if p is None else pd.data_ptr(), dx.data_ptr(), B,
+                                         D, H, W, ci, co, st))
+        r, m = ref[0], mag[0]
+        slack = 0.0
+        if p is not None:
+            q = p.double().requires_grad_(True)
+            Fnn.gelu(q, approximate="tanh").sum().backward()
+            # the derivative through the hardware exp and reciprocal: 1e-5
+            # absolute, as the elementwise kernel's test allows
+            slack = 1e-5 * m
+            r, m = r * q.grad, m * q.grad.abs()
+        err = (dx.double().cpu() - r).abs()
+        assert bool((err <= (27 * co + 2) * EPS * m + slack).all())
+
+
+def test_wgrad_work_is_checked(gpu):
+    from cucim_amd import _array
+    from cucim_amd import _lib as L
+
+    lib = L.lib()
+    x = torch.zeros((1, 3, 3, 3, 24), dtype=torch.bfloat16, device="cuda")
+    f = torch.zeros(27 * 24 * 24 + 24, device="cuda")
+    n = lib.hc_cnn3d_wgrad_work(24, 24)
+    assert lib.hc_cnn3d_wgrad_work(24, 8) < 0
+    for elems, ptr in ((n - 1, f.data_ptr()), (n, f.data_ptr() + 4)):
+        rc = lib.hc_cnn3d_wgrad_batch(x.data_ptr(), f.data_ptr(), f.data_ptr(), f.data_ptr(), 1, 3,
+                                      3, 3, 24, 24, ptr, elems, _array.stream())
+        assert rc == L.ERR_VALUE
+
+
+def test_step_batches_like_single_patches(gpu, monkeypatch):
+    """Patches of two shapes in one step: stacked, or one by one."""
+    from cucim_amd import surrogate as S
+
+    g = torch.Generator().manual_seed(5)
+    xs = [torch.rand((e, e, e + 1, 1), generator=g).to(torch.bfloat16).cuda()
+          for e in (14, 14, 14, 12, 13)]
+    ts = [torch.rand(tuple(s - 10 for s in x.shape[:3]), generator=g).cuda() for x in xs]
+    got = []
+    for most in (S._BATCH_VOXELS, 1):
+        monkeypatch.setattr(S, "_BATCH_VOXELS", most)
+        assert len(list(S._batches(xs, ts))) == (3 if most > 1 else 5)
+        m = S.FrangiSurrogate(seed=3)
+        loss = m.train_step(xs, ts)
+        got.append((float(loss), [t.clone() for t in m._gw + m._gb]))
+    assert abs(got[0][0] - got[1][0]) <= 1e-5 * got[1][0]
+    for a, b in zip(got[0][1], got[1][1]):
+        assert float((a - b).norm()) <= 1e-5 * float(b.norm())
+    assert np.isfinite(got[0][0])
