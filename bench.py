@@ -384,7 +384,7 @@ def bench_surrogate(steps, edge=512, ntubes=320):
            "surrogate_rel_l2": rel_l2(sur, plain),
            "surrogate_dice": dice(sur, plain, 0.5 * float(plain.max())),
            "tflops_surrogate": 95904 * nvox / (ms_sur * 1e-3) / 1e12,
-           "conv_traffic_bytes_per_launch": read_traffic("k_conv3d_mfma",
+           "conv_traffic_bytes_per_launch": read_traffic("k_conv3d_24x24",
                                                          "surrogate_512cubed_counters.txt")}
     del sur
     cs = CheckedSurrogate(model, shape, brick=64, tol=0.02)

@@ -31,6 +31,41 @@ def _grads(x, w, dy):
     return x.grad, w.grad, b.grad
 
 
+@pytest.mark.parametrize("ci,co,act", [(24, 24, 1), (1, 24, 1), (24, 1, 0), (24, 1, 2)])
+@pytest.mark.parametrize("shape", [(2, 3, 3, 3), (3, 5, 11, 19), (3, 29, 59, 117)])
+def test_batched_forward(gpu, ci, co, act, shape):
+    """Batches through both block heights (the last shape has enough blocks
+    for eight planes), one element past 16-byte alignment on the output."""
+    from cucim_amd import _array
+    from cucim_amd import _lib as L
+
+    lib, st = L.lib(), _array.stream()
+    g = torch.Generator().manual_seed(7)
+    x = torch.randn(shape + (ci,), generator=g).to(torch.bfloat16)
+    w = torch.randn((27, ci, co), generator=g) / (27 * ci) ** 0.5
+    b = torch.randn(co, generator=g) * 0.1
+    wq = w.to(torch.bfloat16).double()
+    ref = _conv(x.double(), wq, b.double())
+    mag = _conv(x.double().abs(), wq.abs(), b.double().abs())
+    out_t = torch.bfloat16 if co == 24 else torch.float32
+    out = torch.empty(ref.numel() + 1, dtype=out_t, device="cuda")[1:].view(ref.shape)
+    pre = torch.empty(ref.numel() + 1, device="cuda")[1:].view(ref.shape)
+    wd, bd, xd = w.cuda(), b.cuda(), x.cuda()
+    packed = torch.empty(lib.hc_cnn3d_packed_size(ci, co), dtype=torch.uint8, device="cuda")
+    L.check(lib.hc_cnn3d_pack(wd.data_ptr(), packed.data_ptr(), ci, co, st))
+    L.check(lib.hc_cnn3d_conv(_array.hc_array(xd), _array.hc_array(out), packed.data_ptr(),
+                              bd.data_ptr(), act, pre.data_ptr(), st))
+    p = pre.double().cpu()
+    # the products of bfloat16 values are exact in float32
+    assert bool(((p - ref).abs() <= (27 * ci + 1) * EPS * mag).all())
+    if act == 1:
+        # the hardware exp and reciprocal (1e-6 relative), then one bf16 rounding
+        exp = Fnn.gelu(p, approximate="tanh")
+        assert bool(((out.double().cpu() - exp).abs() <= 2.0 ** -8 * exp.abs() + 1e-5).all())
+    else:
+        assert torch.equal(out.cpu(), (pre.clamp(0, 1) if act == 2 else pre).cpu())
+
+
 @pytest.mark.parametrize("ci,co", [(24, 24), (1, 24), (24, 1)])
 @pytest.mark.parametrize("shape", [(1, 3, 3, 3), (2, 4, 10, 18), (3, 5, 11, 19), (1, 20, 3, 35),
                                    (2, 13, 27, 9)])
