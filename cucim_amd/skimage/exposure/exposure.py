@@ -66,19 +66,20 @@ def _dtype_limits(dt):
     return int(info.min), int(info.max)
 
 
-def _histogram_flat(x, nbins, source_range, normalize):
-    """``_histogram`` (:308-345) of a flattened C-contiguous tensor."""
+def _histogram_flat(x, nbins, source_range, normalize, rng=None):
+    """``_histogram`` (:308-345) of a flattened C-contiguous tensor.  rng: its
+    (min, max) where the caller has it already."""
     dt = _array.np_dtype(x.dtype)
     if source_range not in ("image", "dtype"):
         raise ValueError(f"Incorrect value for `source_range` argument: {source_range}")
     if dt.kind in "iub":
         # bincount over [min, max] (image) or the dtype's range (:51-105)
-        lo, hi = _range(x) if source_range == "image" else _dtype_limits(dt)
+        lo, hi = (rng or _range(x)) if source_range == "image" else _dtype_limits(dt)
         counts = _counts(x, hi - lo + 1, None, lo)
         centers = torch.arange(lo, hi + 1, dtype=torch.int64, device=x.device)
     else:
         if source_range == "image":
-            first, last = _range(x) if x.numel() else (0.0, 1.0)
+            first, last = (rng or _range(x)) if x.numel() else (0.0, 1.0)
         else:
             first, last = (-1.0, 1.0)
         e = _float_edges(first, last, int(nbins), dt)

@@ -16,7 +16,7 @@ import numpy as np
 import torch
 
 from ... import _array, _lib, _trace
-from ..exposure.exposure import _range, histogram
+from ..exposure.exposure import _histogram_flat, _range
 
 __all__ = ["threshold_otsu", "threshold_yen", "threshold_li"]
 
@@ -29,11 +29,11 @@ def _scalar(v, like_dtype=None):
     return torch.from_numpy(np.array(a)).to(_array.device())
 
 
-def _validate_image_histogram(image, hist, nbins=None, normalize=False):
+def _validate_image_histogram(image, hist, nbins=None, normalize=False, rng=None):
     """``thresholding.py:298-352``: counts (float32) and bin centers, from
     ``hist`` (trimmed of leading / trailing empty bins) or the image's
     histogram; returned as host arrays (the reference moves them to the host
-    before the per-bin arithmetic)."""
+    before the per-bin arithmetic).  rng: the image's (min, max) if known."""
     if image is None and hist is None:
         raise Exception("Either image or hist must be provided.")
     if hist is not None:
@@ -49,8 +49,8 @@ def _validate_image_histogram(image, hist, nbins=None, normalize=False):
             end = cond.size - int(np.argmax(cond[::-1]))
             counts, centers = counts[start:end], centers[start:end]
     else:
-        counts, centers = histogram(_array.as_tensor(image).reshape(-1), nbins,
-                                    source_range="image", normalize=normalize)
+        counts, centers = _histogram_flat(_array.as_tensor(image).contiguous().reshape(-1),
+                                          nbins, "image", normalize, rng)
         counts, centers = _host(counts), _host(centers)
     return counts.astype(np.float32, copy=False), centers
 
@@ -59,16 +59,6 @@ def _host(a):
     if isinstance(a, torch.Tensor):
         return a.detach().cpu().numpy()
     return np.asarray(a)
-
-
-def _single_value(image):
-    """(True, value) when every element equals the first one (the
-    reference's ``cp.all(image == first_pixel)``), via the device range."""
-    x = _array.as_tensor(image).contiguous().reshape(-1)
-    lo, hi = _range(x)
-    if lo == hi:  # NaN compares unequal
-        return True, x[0].clone()
-    return False, None
 
 
 def _otsu_from_hist(counts, centers):
@@ -92,10 +82,15 @@ def threshold_otsu(image=None, nbins=256, *, hist=None):
             warn(f"threshold_otsu is expected to work correctly only for grayscale images; "
                  f"image shape {tuple(image.shape)} looks like that of an RGB image.",
                  stacklevel=2)
-        same, v = _single_value(image)
-        if same:
-            return v
-    counts, centers = _validate_image_histogram(image, hist, nbins)
+        # every element equal to the first one (the reference's
+        # ``cp.all(image == first_pixel)``): the range is one value (NaN
+        # compares unequal)
+        image = image.contiguous().reshape(-1)
+        rng = _range(image)
+        if rng[0] == rng[1]:
+            return image[0].clone()
+    counts, centers = _validate_image_histogram(image, hist, nbins,
+                                                rng=None if image is None else rng)
     with np.errstate(divide="ignore", invalid="ignore"):
         return _scalar(_otsu_from_hist(counts, centers))
 
