@@ -121,7 +121,11 @@ __global__ __launch_bounds__(256) void k_meij_vals(const SArgs<W> a, W* __restri
       red[threadIdx.x] = red[threadIdx.x + s];
     __syncthreads();
   }
-  if (threadIdx.x == 0) atomicMax(mx, red[0]);
+  // atomics on one word are done one after another: none where the maximum
+  // seen (perhaps an older, smaller one) is at least as large
+  if (threadIdx.x == 0 &&
+      red[0] > __hip_atomic_load(mx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP))
+    atomicMax(mx, red[0]);
 }
 
 template <typename W>
