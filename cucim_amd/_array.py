@@ -93,10 +93,9 @@ def hc_array(t):
     a = _lib.HCArray()
     a.data = t.data_ptr()
     a.dtype = _TORCH_TO_HC[t.dtype]
-    a.ndim = t.dim()
-    for d in range(t.dim()):
-        a.shape[d] = t.shape[d]
-        a.strides[d] = t.stride(d)
+    a.ndim = n = t.dim()
+    a.shape[:n] = t.shape
+    a.strides[:n] = t.stride()
     return a
 
 
@@ -108,7 +107,9 @@ def hc_arrays(ts):
 
 
 def stream():
-    return torch.cuda.current_stream().cuda_stream
+    """The current stream's handle, without the Stream object that
+    torch.cuda.current_stream() builds (5 us a call)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def empty(shape, dtype):

@@ -233,10 +233,11 @@ def load_library(path=LIB_PATH):
 
 
 def lib():
-    """The loaded library, for compute calls: requires a visible GPU."""
+    """The loaded library, for compute calls: requires a visible GPU (torch's
+    runtime, once initialised, has one)."""
     import torch
 
-    if not torch.cuda.is_available():
+    if not torch.cuda.is_initialized() and not torch.cuda.is_available():
         raise RuntimeError("cucim_amd needs a ROCm GPU; none is visible")
     return load_library()
 

@@ -1,6 +1,7 @@
 """Hessian matrix and its eigenvalues (``feature/corner.py`` of the
 reference, paths relative to ``python/cucim/src/cucim/skimage/``)."""
 
+import functools
 import math
 from itertools import combinations_with_replacement
 from warnings import warn
@@ -57,6 +58,14 @@ def _taps_arrays(kernels, f64):
     return ts, td, keep
 
 
+@functools.lru_cache(maxsize=32)
+def _hessian_taps(sigma, ndim, dtype_str):
+    """The tap arrays of one Hessian, shared by the calls of one (sigma, ndim,
+    dtype)."""
+    dtype = np.dtype(dtype_str)
+    return _taps_arrays(hessian_kernels(sigma, ndim, dtype), dtype == np.float64)
+
+
 def _hessian_sequential(image, sigma, mode, cval, order):
     """The reference's pass sequence (``corner.py:218-254``) on the tiled
     line kernels; used when the fused schedule does not fit."""
@@ -93,8 +102,11 @@ def _hessian_matrix_with_gaussian(image, sigma=1, mode="reflect", cval=0, order=
         x = image.contiguous()
         nH = ndim * (ndim + 1) // 2
         H = [_array.empty(x.shape, float_dtype) for _ in range(nH)]
-        f64 = float_dtype == np.float64
-        ts, td, keep = _taps_arrays(hessian_kernels(sigma, ndim, float_dtype), f64)
+        sg = (sigma,) * ndim if np.isscalar(sigma) else tuple(sigma)
+        # numpy scalars bring their own precision into the kernels: not cached
+        taps = _hessian_taps if all(type(v) in (int, float) for v in sg) \
+            else _hessian_taps.__wrapped__
+        ts, td, _keep = taps(sg, ndim, np.dtype(float_dtype).str)
         scratch = torch.empty(64, dtype=torch.uint8, device=x.device)
         rc = _lib.lib().hc_hessian_gaussian(
             _array.hc_array(x), _array.hc_arrays(H), nH, ts, td, _mode_code(mode),
