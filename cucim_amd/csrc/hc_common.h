@@ -257,20 +257,23 @@ __device__ __forceinline__ W roundtrip(W v, int dt) {
 // Boundary extension of position p on an axis of length n,
 // _vendored/_ndimage_util.py:186-308.  Returns -1 for constant mode outside
 // the array.  In-range positions return unchanged.
-__device__ __host__ __forceinline__ int64_t remap(int64_t p, int64_t n, int mode) {
+// I: int64_t, or int where every position fits (a 64-bit remainder takes the
+// GPU some 60 instructions).
+template <typename I>
+__device__ __host__ __forceinline__ I remap_as(I p, I n, int mode) {
   if (p >= 0 && p < n) return p;
   switch (mode) {
     case HC_MODE_REFLECT: {  // i<0 -> -1-i; i %= 2n; i = min(i, 2n-1-i)
       if (p < 0) p = -1 - p;
       p %= 2 * n;
-      int64_t q = 2 * n - 1 - p;
+      I q = 2 * n - 1 - p;
       return p < q ? p : q;
     }
     case HC_MODE_MIRROR: {  // n==1 -> 0; i<0 -> -i; 1 + (i-1) % (2n-2); min(i, 2n-2-i)
       if (n == 1) return 0;
       if (p < 0) p = -p;
       p = 1 + (p - 1) % (2 * n - 2);
-      int64_t q = 2 * n - 2 - p;
+      I q = 2 * n - 2 - p;
       return p < q ? p : q;
     }
     case HC_MODE_NEAREST:
@@ -282,6 +285,10 @@ __device__ __host__ __forceinline__ int64_t remap(int64_t p, int64_t n, int mode
     default:
       return -1;
   }
+}
+
+__device__ __host__ __forceinline__ int64_t remap(int64_t p, int64_t n, int mode) {
+  return remap_as<int64_t>(p, n, mode);
 }
 
 // Work-groups are dispatched round-robin over the 8 XCDs (block b runs on XCD

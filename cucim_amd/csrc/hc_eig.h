@@ -76,6 +76,53 @@ __device__ __forceinline__ void sincos_small(double t, double& c, double& s) {
   s = fma(ps * z, t, t);
 }
 
+// 1 / sqrt(x) for normal positive x, to about an ulp of double: the hardware
+// estimate (24 bits) and one third-order step.
+__device__ __forceinline__ double rsqrt_fast(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
+// cos(phi / 3) and sin(phi / 3) of the angle phi in [0, pi] with cosine c and
+// sine s (doubles): the angle in float, then one Newton step for w^3 = c + i s
+// on the unit circle, w1 = (2 w0 + z conj(w0)^2 / |w0|^4) / 3, whose error is
+// the square of w0's (3e-7 at most): 1e-13 against 1e-16 of a double arctangent
+// and its sine and cosine, which took twice the instructions; the float
+// rounding of the eigenvalues is 6e-8.  atan(t) on [0, 1] by the minimax-like
+// odd polynomial of Abramowitz & Stegun 4.4.49 (2e-8); the sine and cosine by
+// their Taylor series on [0, pi / 3].
+__device__ __forceinline__ void third_angle(double c, double s, double& ct, double& st) {
+  const float cf = (float)c, sf = (float)s, ca = fabsf(cf);
+  const float hi = fmaxf(ca, sf), lo = fminf(ca, sf);
+  const float t = lo * __builtin_amdgcn_rcpf(hi), z = t * t;
+  float p = fmaf(z, 0.0028662257f, -0.0161657367f);
+  p = fmaf(p, z, 0.0429096138f);
+  p = fmaf(p, z, -0.0752896400f);
+  p = fmaf(p, z, 0.1065626393f);
+  p = fmaf(p, z, -0.1420889944f);
+  p = fmaf(p, z, 0.1999355085f);
+  p = fmaf(p, z, -0.3333314528f);
+  float phi = fmaf(t * z, p, t);
+  if (sf > ca) phi = 1.57079632679f - phi;
+  if (cf < 0.f) phi = 3.14159265359f - phi;
+  const float th = phi * 0.333333333f, q = th * th;
+  float k = fmaf(q, -2.7557319e-7f, 2.4801587e-5f);
+  k = fmaf(k, q, -1.3888889e-3f);
+  k = fmaf(k, q, 4.1666667e-2f);
+  k = fmaf(k, q, -0.5f);
+  float m = fmaf(q, -2.5052108e-8f, 2.7557319e-6f);
+  m = fmaf(m, q, -1.9841270e-4f);
+  m = fmaf(m, q, 8.3333333e-3f);
+  m = fmaf(m, q, -0.16666667f);
+  const double c0 = (double)fmaf(k, q, 1.f), s0 = (double)fmaf(m * q, th, th);
+  const double cc = c0 * c0, ss = s0 * s0, f = fma(-2.0, cc + ss, 3.0);  // 1 / |w0|^4
+  const double u = f * (cc - ss), v = -2.0 * f * (c0 * s0);              // conj(w0)^2 / |w0|^4
+  constexpr double third = 1.0 / 3.0;
+  ct = third * fma(2.0, c0, fma(c, u, -s * v));
+  st = third * fma(2.0, s0, fma(c, v, s * u));
+}
+
 // 3x3, Deledalle et al. (2017) closed form in double (corner.py:566-612) for
 // the matrix [[a, d, f], [d, b, e], [f, e, c]], then the reference's three
 // compare-swap steps (corner.py:613-647).  With abs_sort the comparison keys
@@ -94,23 +141,36 @@ __device__ __forceinline__ void eig33(F aa, F bb, F cc, F dd, F ee, F ff, int de
   x2 -= 54 * (d * e * f);
   double x1 = a * a + b * b + c * c - a * b - a * c - b * c + 3 * (d_sq + e_sq + f_sq);
   x1 = fmax(x1, 0.0);
-  double phi;
-  if (x2 == 0.0) {
-    phi = M_PI / 2.0;
-  } else {
-    const double arg = fmax(4 * x1 * x1 * x1 - x2 * x2, 0.0);
-    phi = atan(sqrt(arg) / x2);
-    if (x2 < 0) phi += M_PI;
-  }
   // the reference divides by 3; a product with the double nearest 1/3
   // differs by at most an ulp of double, far below the float rounding that
   // follows, and avoids four IEEE divisions
   constexpr double third = 1.0 / 3.0;
-  const double x1_term = (2.0 / 3.0) * sqrt(x1);
   const double abc = (a + b + c) * third;
-  // cos(phi / 3), cos((phi - pi) / 3), cos((phi + pi) / 3)
-  double ct, st;
-  sincos_small(phi * third, ct, st);
+  // x1_term = (2 / 3) sqrt(x1); cos(phi / 3), sin(phi / 3), from which
+  // cos((phi - pi) / 3) and cos((phi + pi) / 3)
+  double x1_term, ct, st;
+  if constexpr (sizeof(F) == 4) {
+    // cos(phi) = x2 / (2 x1^(3/2)); x1 of floats is 0 or at least 1e-91.  With
+    // x1 = 0 every x2 but NaN gives phi = pi / 2, as below.  An infinite x1
+    // (from infinite elements of opposite signs) gives NaN.
+    const double y = x1 > 1e-200 ? rsqrt_fast(x1) : 0.0;
+    x1_term = (2.0 / 3.0) * (x1 * y);
+    const double cp = x2 * (0.5 * y * y * y);
+    const double s2 = fmax(fma(-cp, cp, 1.0), 0.0);
+    const double sp = s2 > 1e-200 ? s2 * rsqrt_fast(s2) : 0.0;
+    third_angle(cp, sp, ct, st);
+  } else {
+    double phi;
+    if (x2 == 0.0) {
+      phi = M_PI / 2.0;
+    } else {
+      const double arg = fmax(4 * x1 * x1 * x1 - x2 * x2, 0.0);
+      phi = atan(sqrt(arg) / x2);
+      if (x2 < 0) phi += M_PI;
+    }
+    x1_term = (2.0 / 3.0) * sqrt(x1);
+    sincos_small(phi * third, ct, st);
+  }
   const double half_c = 0.5 * ct, r3_s = 0.86602540378443864676 * st;  // sqrt(3) / 2
   F lam1 = (F)(abc - x1_term * ct);
   F lam2 = (F)(abc + x1_term * (half_c + r3_s));
@@ -217,19 +277,33 @@ __device__ __forceinline__ F frangi_v3r(F l1, F l2, F l3, F r_g, const FrangiNeg
 }
 
 // float32 forms of the two above, used by the fused float32 passes: the
-// exponentials in float (1 - e^x as -expm1(x), accurate where x is small)
+// exponentials in float (1 - e^x accurate where x is small)
 // instead of double.  The result then differs from the reference's
 // double-then-round value by a few float ulps (each exponential within about
 // an ulp of its argument's relative error, one float rounding per product),
 // far below the rounding of the float32 Hessian the vesselness is built
 // from; it saves the three double exponentials per voxel and sigma.
+// 1 - e^x for x <= 0 (NaN passes): the Taylor series where the difference
+// cancels, else from the hardware exponential; within 2 ulp.
+__device__ __forceinline__ float one_minus_exp(float x) {
+  float p = fmaf(x, 1.f / 40320.f, 1.f / 5040.f);
+  p = fmaf(p, x, 1.f / 720.f);
+  p = fmaf(p, x, 1.f / 120.f);
+  p = fmaf(p, x, 1.f / 24.f);
+  p = fmaf(p, x, 1.f / 6.f);
+  p = fmaf(p, x, 0.5f);
+  p = -fmaf(p * x, x, x);
+  const float e = 1.f - __builtin_amdgcn_exp2f(x * 1.44269504f);
+  return x > -0.5f ? p : e;
+}
+
 template <>
 __device__ __forceinline__ float frangi_v2r<float>(float l1, float l2, float r_g,
                                                    const FrangiNegRecip& q) {
   float r_b = fabsf(l1) / fmaxf(l2, 1.0e-10f);
   r_b *= r_b;
   const float result = expf(r_b * (float)q.b);
-  return result * -expm1f(r_g * (float)q.g);
+  return result * one_minus_exp(r_g * (float)q.g);
 }
 
 template <>
@@ -240,9 +314,9 @@ __device__ __forceinline__ float frangi_v3r<float>(float l1, float l2, float l3,
   float r_a = lam2 / lam3;
   r_a *= r_a;
   const float r_b = (l1 * l1) / (lam2 * lam3);
-  float result = -expm1f(r_a * (float)q.a);
+  float result = one_minus_exp(r_a * (float)q.a);
   result *= expf(r_b * (float)q.b);
-  return result * -expm1f(r_g * (float)q.g);
+  return result * one_minus_exp(r_g * (float)q.g);
 }
 
 // cp.maximum: NaN-propagating

@@ -311,20 +311,24 @@ __device__ __forceinline__ void chain_pass_mfma(f32x4_t (&acc)[NS][NBW], const f
   }
   // blocks past the last are computed on the last one's rows (no branch in
   // the loop); their results are never stored
-  int rb[NBW];
+  const float* pb[NBW];
 #pragma unroll
-  for (int i = 0; i < NBW; ++i) rb[i] = (min(wv + NW * i, nblk - 1) * 16 + kk) * ps + ii * ls;
+  for (int i = 0; i < NBW; ++i)
+    pb[i] = X + (min(wv + NW * i, nblk - 1) * 16 + kk) * ps + ii * ls;
+  const float* pa[NS];
+#pragma unroll
+  for (int s = 0; s < NS; ++s) pa[s] = wp[s] + 15 + kk - ii;
   // Software-pipelined over two operand sets: the operands of step st + 1
   // are read from LDS while the products of step st run, so no product
-  // waits for its own reads (a read past the last step re-reads the last
-  // step's operands, which are then unused).
-  const int w0 = 15 + kk - ii, last = nsteps - 1;
+  // waits for its own reads.  The pointers move once per two steps, the reads
+  // between are at constant offsets.  The read past the last step touches at
+  // most four rows (words of the taps) past those the passes need, which lie
+  // within the work-group's LDS, and is unused.
   auto fetch = [&](float (&a)[NS], float (&b)[NBW], int st) {
-    const int t = min(st, last);
 #pragma unroll
-    for (int s = 0; s < NS; ++s) a[s] = wp[s][w0 + 4 * t];
+    for (int s = 0; s < NS; ++s) a[s] = pa[s][4 * st];
 #pragma unroll
-    for (int i = 0; i < NBW; ++i) b[i] = X[rb[i] + 4 * t * ps];
+    for (int i = 0; i < NBW; ++i) b[i] = pb[i][4 * st * ps];
   };
   auto step = [&](const float (&a)[NS], const float (&b)[NBW]) {
 #pragma unroll
@@ -337,9 +341,13 @@ __device__ __forceinline__ void chain_pass_mfma(f32x4_t (&acc)[NS][NBW], const f
   fetch(a0, b0, 0);
   int st = 0;
   for (; st + 1 < nsteps; st += 2) {
-    fetch(a1, b1, st + 1);
+    fetch(a1, b1, 1);
     step(a0, b0);
-    fetch(a0, b0, st + 2);
+    fetch(a0, b0, 2);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) pa[s] += 8;
+#pragma unroll
+    for (int i = 0; i < NBW; ++i) pb[i] += 8 * ps;
     step(a1, b1);
   }
   if (st < nsteps) step(a0, b0);  // an odd step count's last step
@@ -412,8 +420,8 @@ __device__ __forceinline__ void halo_table(short* hsrc, int E, int64_t N, int sh
   const int nh = E - (int)N;
   for (int h = tid; h < nh; h += nt) {
     const int q = h < shift ? h : h + (int)N;
-    const int64_t r = remap((int64_t)q - shift, N, mode);
-    hsrc[h] = (short)(r >= 0 ? (int)r + shift : -1);
+    const int r = remap_as<int>(q - shift, (int)N, mode);
+    hsrc[h] = (short)(r >= 0 ? r + shift : -1);
   }
 }
 
@@ -429,6 +437,12 @@ __device__ __forceinline__ void fill_halo(float* X, float* Y, int E, int N, int 
     X[q * ps + c * ls] = src >= 0 ? X[src * ps + c * ls] : cval;
     if (Y) Y[q * ps + c * ls] = src >= 0 ? Y[src * ps + c * ls] : cval;
   }
+}
+
+// L / inner; 32-bit where the lines' number allows (a 64-bit division takes
+// the vector ALU some 100 instructions).
+__device__ __forceinline__ int64_t outer_of(int64_t L, int64_t inner, int64_t nlines) {
+  return nlines <= 0x7fffffff ? (int64_t)((unsigned)L / (unsigned)inner) : L / inner;
 }
 
 // Stages (tile, job) per work-group of the matrix-core chain pass.
@@ -461,7 +475,7 @@ k_chain_mfma(const ChainArgs<float> a) {
     const int64_t L = (st - job * ntile) * kChC + cs;
     const ChainJob& jb = a.job[job];
     const bool ok = L < nlines;
-    const int64_t lo = ok ? L / inner : 0, li = ok ? L - lo * inner : 0;
+    const int64_t lo = ok ? outer_of(L, inner, nlines) : 0, li = ok ? L - lo * inner : 0;
     const int64_t base = lo * N * inner + li;
     if (jb.in_dt == HC_FLOAT32) {
       // All NPF loads are issued before any is waited for: every load is
@@ -474,11 +488,13 @@ k_chain_mfma(const ChainArgs<float> a) {
       const bool neg = a.negate != 0;
       const bool ctr = a.center != nullptr;
       const float c = ctr ? (float)*a.center : 0.f;
+      const float* in0 = in + base + (int64_t)ns0 * inner;
 #pragma unroll
       for (int u = 0; u < NPF; ++u) {
+        // rows that every thread has take a uniform offset
         const int n = ns0 + 4 * NW * u;
-        const bool use = ok && n < N;
-        v[u] = in[base + (use ? (int64_t)n : 0) * inner];
+        v[u] = 4 * NW * (u + 1) <= N ? in0[(int64_t)(4 * NW * u) * inner]
+                                     : in[base + (n < N ? (int64_t)n : 0) * inner];
       }
 #pragma unroll
       for (int u = 0; u < NPF; ++u) {
@@ -509,16 +525,14 @@ k_chain_mfma(const ChainArgs<float> a) {
     const int job = (int)(st / ntile);
     const int64_t L0 = (st - job * ntile) * kChC;
     const ChainJob& jb = a.job[job];
-    bool bad = false;
+    float chk = 0.f;  // stays 0 while every value is finite
 #pragma unroll
     for (int u = 0; u < NPF; ++u) {
       const int n = ns0 + 4 * NW * u;
-      if (n < N) {
-        bufA[(shift + n) * kMfS + cs] = pf[u];
-        bad |= !finite(pf[u]);
-      }
+      if (n < N) bufA[(shift + n) * kMfS + cs] = pf[u];
+      chk = fmaf(pf[u], 0.f, chk);
     }
-    const bool skip0 = __syncthreads_or(bad) || cval_bad;
+    const bool skip0 = __syncthreads_or(!(chk == 0.f)) || cval_bad;
     // the work-group's next stage is in flight during this one's passes
     if (st + 1 < nst && st + 1 < st0 + kChainSPW) load(pf, st + 1);
     fill_halo(bufA, nullptr, E, (int)N, shift, hsrc, a.cval, tid, NT);
@@ -544,16 +558,16 @@ k_chain_mfma(const ChainArgs<float> a) {
       }
     }
     __syncthreads();  // every read of the staged input is done
-    bool bad1 = false;
+    float chk1 = 0.f;
 #pragma unroll
     for (int i = 0; i < NBW; ++i) {
       if (wv + NW * i >= nblk) continue;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) bad1 |= !(finite(f[0][i][r]) && finite(f[1][i][r]));
+      for (int r = 0; r < 4; ++r) chk1 = fmaf(f[1][i][r], 0.f, fmaf(f[0][i][r], 0.f, chk1));
     }
     const int64_t L = L0 + ii;
     const bool lok = L < nlines;
-    const int64_t lo = lok ? L / inner : 0, li = lok ? L - lo * inner : 0;
+    const int64_t lo = lok ? outer_of(L, inner, nlines) : 0, li = lok ? L - lo * inner : 0;
     const int64_t base = lo * N * inner + li;
     // second passes, per first op: its results go through the one line
     // buffer in turn (the other op's results wait in registers)
@@ -575,7 +589,7 @@ k_chain_mfma(const ChainArgs<float> a) {
         for (int r = 0; r < 4; ++r) bufA[(shift + 16 * b + 4 * kk + r) * kMfS + ii] = f[src][i][r];
       }
       if (first_src)
-        skip1 = __syncthreads_or(bad1) || skip0;
+        skip1 = __syncthreads_or(!(chk1 == 0.f)) || skip0;
       else
         __syncthreads();
       first_src = false;
@@ -595,22 +609,28 @@ k_chain_mfma(const ChainArgs<float> a) {
           y[1][i] = g[0][i];
         }
       }
-      float* os = ks >= 0 ? reinterpret_cast<float*>(jb.o[ks].out) : nullptr;
-      float* od = kd >= 0 ? reinterpret_cast<float*>(jb.o[kd].out) : nullptr;
-      if (lok) {
+      // this lane's line from position 4 kk; the offsets from there are
+      // uniform, and only a line's last block needs a mask
+      const int64_t lane0 = base + (int64_t)(4 * kk) * inner;
+      auto store = [&](void* out, const f32x4_t (&v)[NBW]) {
+        float* o = reinterpret_cast<float*>(out) + lane0;
 #pragma unroll
         for (int i = 0; i < NBW; ++i) {
           const int b = wv + NW * i;
           if (b >= nblk) continue;
+          if (16 * b + 16 <= N) {
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int64_t n = 16 * b + 4 * kk + r;
-            if (n < N) {
-              if (os) os[base + n * inner] = y[0][i][r];
-              if (od) od[base + n * inner] = y[1][i][r];
-            }
+            for (int r = 0; r < 4; ++r) o[(int64_t)(16 * b + r) * inner] = v[i][r];
+          } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              if (16 * b + 4 * kk + r < N) o[(int64_t)(16 * b + r) * inner] = v[i][r];
           }
         }
+      };
+      if (lok) {
+        if (ks >= 0) store(jb.o[ks].out, y[0]);
+        if (kd >= 0) store(jb.o[kd].out, y[1]);
       }
     }
     __syncthreads();  // the buffers are restaged for the next stage
@@ -950,7 +970,7 @@ __device__ __forceinline__ bool final_stage(const FinalArgs<float>& a, const Fin
   const bool rok = row < g.nrows;
   const float* rp = a.in[J] + (rok ? row : 0) * g.N;
   float* xl = X + l * LS + g.shift;
-  bool bad = false;
+  float chk = 0.f;  // stays 0 while every value is finite
   if (a.vec4) {
     // N <= 16 NW NBW, so a line has at most NBW CS chunks
     F4 v[NBW];
@@ -964,7 +984,7 @@ __device__ __forceinline__ bool final_stage(const FinalArgs<float>& a, const Fin
       const int c = c0 + CS * k;
       if (4 * c >= n) continue;
       const F4 w = rok ? v[k] : F4{0.f, 0.f, 0.f, 0.f};
-      bad |= !(finite(w[0]) && finite(w[1]) && finite(w[2]) && finite(w[3]));
+      chk = fmaf(w[3], 0.f, fmaf(w[2], 0.f, fmaf(w[1], 0.f, fmaf(w[0], 0.f, chk))));
       *reinterpret_cast<F2*>(xl + 4 * c) = F2{w[0], w[1]};
       *reinterpret_cast<F2*>(xl + 4 * c + 2) = F2{w[2], w[3]};
     }
@@ -980,11 +1000,11 @@ __device__ __forceinline__ bool final_stage(const FinalArgs<float>& a, const Fin
       const int q = c0 + CS * k;
       if (q >= n) continue;
       const float w = rok ? v[k] : 0.f;
-      bad |= !finite(w);
+      chk = fmaf(w, 0.f, chk);
       xl[q] = w;
     }
   }
-  return bad;
+  return !(chk == 0.f);
 }
 
 // Input J of the tile: stage it, first op, re-extend, second op into res.
@@ -1007,7 +1027,7 @@ __device__ __forceinline__ void final_input_mfma(const FinalArgs<float>& a, cons
     const float* const wp[1] = {a.first[J] ? wpD : wpS};
     chain_pass<NBW, 1, NW>(skip0, f, xin, wp, g.Km, g.nd, g.nblk, wv, lane, 1, LS);
   }
-  bool bad1 = false;
+  float chk1 = 0.f;
 #pragma unroll
   for (int i = 0; i < NBW; ++i) {
     if (wv + NW * i >= g.nblk) continue;
@@ -1016,9 +1036,9 @@ __device__ __forceinline__ void final_input_mfma(const FinalArgs<float>& a, cons
     *reinterpret_cast<F2*>(d) = F2{f[0][i][0], f[0][i][1]};
     *reinterpret_cast<F2*>(d + 2) = F2{f[0][i][2], f[0][i][3]};
 #pragma unroll
-    for (int r = 0; r < 4; ++r) bad1 |= !finite(f[0][i][r]);
+    for (int r = 0; r < 4; ++r) chk1 = fmaf(f[0][i][r], 0.f, chk1);
   }
-  const bool skip1 = __syncthreads_or(bad1) || skip0;
+  const bool skip1 = __syncthreads_or(!(chk1 == 0.f)) || skip0;
   fill_halo(xf, nullptr, E, (int)g.N, shift, hsrc, a.cval, tid, NT, 1, LS);
   __syncthreads();
   {
@@ -1157,11 +1177,14 @@ __global__ __launch_bounds__(256) void k_frangi_from_eig(const W* __restrict__ e
                                                          double alpha_sq, double beta_sq,
                                                          const double* gamma_sq_dev) {
   const double gsq = *gamma_sq_dev;
+  const FrangiNegRecip nrc = frangi_neg_recip(alpha_sq, beta_sq, gsq);
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * 256) {
     if (NDIM == 3) {
-      const W l1 = e0[i], l2 = e1[i], l3 = e2[i];
-      out[i] = frangi_v3<W>(l1, l2, l3, frangi_rg3<W>(l1, l2, l3), alpha_sq, beta_sq, gsq);
+      // float: as the final pass computes the later sigmas
+      const W l1 = e0[i], l2 = e1[i], l3 = e2[i], rg = frangi_rg3<W>(l1, l2, l3);
+      out[i] = sizeof(W) == 4 ? frangi_v3r<W>(l1, l2, l3, rg, nrc)
+                              : frangi_v3<W>(l1, l2, l3, rg, alpha_sq, beta_sq, gsq);
     } else {
       const W l1 = e0[i], l2 = e1[i];
       out[i] = frangi_v2<W>(l1, l2, frangi_rg2<W>(l1, l2), beta_sq, gsq);
@@ -1316,9 +1339,10 @@ inline bool mfma_geom(const TapPack<float>& S, const TapPack<float>& D, int64_t 
   g.nd = (g.Km + 30) / 16;
   // nbuf line buffers (line-major: 16 lines of lm_stride(E) and two words
   // of alignment room), the padded taps, the halo source rows (16-bit, one
-  // per row outside [shift, shift + N))
+  // per row outside [shift, shift + N)), room for the taps' read past the
+  // last step
   const int buf = line_major ? 2 + nbuf * kChC * lm_stride(g.E) : nbuf * g.E * kMfS;
-  g.lds = (buf + 2 * mfma_wp(g.Km)) * (int)sizeof(float) + ((int)(g.E - N) + 1) / 2 * 4;
+  g.lds = (buf + 2 * mfma_wp(g.Km)) * (int)sizeof(float) + ((int)(g.E - N) + 1) / 2 * 4 + 16;
   return g.lds <= kMaxLds;
 }
 

@@ -1,0 +1,59 @@
+"""Float32 3 x 3 eigenvalues (angle by float estimate and one Newton step)
+against numpy in float64, over magnitudes from denormal cubes to 1e15 and the
+cases where two or three eigenvalues meet; and the float vesselness of the
+first sigma at small and large exponents.
+
+The result is rounded to float32 once (2^-24 of itself); the closed form in
+double adds 1e-13 of the largest eigenvalue, and sqrt(2^-52) = 1.5e-8 of it
+where two eigenvalues meet (the sine of the angle is the root of a rounded
+difference): 2^-23 of the largest eigenvalue bounds both."""
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _matrices(kind, n, rng):
+    if kind == "random":
+        m = rng.standard_normal((n, 3, 3))
+    elif kind == "rank1":
+        v = rng.standard_normal((n, 3))
+        m = v[:, :, None] * v[:, None, :]
+    elif kind == "pair":  # two equal eigenvalues, rotated
+        q = np.linalg.qr(rng.standard_normal((n, 3, 3)))[0]
+        d = np.stack([np.ones(n), np.ones(n), rng.uniform(-2, 2, n)], 1)
+        m = q @ (d[:, :, None] * q.transpose(0, 2, 1))
+    elif kind == "diagonal":
+        m = np.stack([np.diag(v) for v in rng.integers(-2, 3, (n, 3)).astype(float)])
+    else:  # traceless: eigenvalues of opposite sign
+        m = rng.standard_normal((n, 3, 3))
+        m -= np.eye(3) * np.trace(m, axis1=1, axis2=2)[:, None, None] / 3
+    return m + m.transpose(0, 2, 1)
+
+
+@pytest.mark.parametrize("scale", [1e-30, 1e-12, 1.0, 1e6, 1e15])
+@pytest.mark.parametrize("kind", ["random", "rank1", "pair", "diagonal", "traceless"])
+def test_eigenvalues_against_double(gpu, kind, scale):
+    from cucim_amd.skimage.feature import hessian_matrix_eigvals
+
+    rng = np.random.default_rng(3)
+    m = (_matrices(kind, 999, rng) * scale).astype(np.float32)
+    el = [torch.from_numpy(np.ascontiguousarray(m[:, i, j])).cuda().view(3, 3, 111)
+          for i, j in ((0, 0), (0, 1), (0, 2), (1, 1), (1, 2), (2, 2))]
+    got = hessian_matrix_eigvals(el)
+    got = torch.stack(list(got)).cpu().numpy().reshape(3, -1).astype(np.float64)
+    exp = np.linalg.eigvalsh(m.astype(np.float64))[:, ::-1].T
+    top = np.abs(exp).max(0)
+    assert (np.abs(got - exp) <= 2.0 ** -23 * top + 1e-44).all()
+
+
+def test_eigenvalues_of_zero_and_nan(gpu):
+    from cucim_amd.skimage.feature import hessian_matrix_eigvals
+
+    el = [torch.zeros((2, 2, 2), device="cuda") for _ in range(6)]
+    assert all(bool((v == 0).all()) for v in hessian_matrix_eigvals(el))
+    el[1][0, 0, 0] = float("nan")
+    for v in hessian_matrix_eigvals(el):
+        assert bool(v[0, 0, 0].isnan()) and int(v.isnan().sum()) == 1
