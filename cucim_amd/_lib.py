@@ -44,6 +44,7 @@ ENTRY_POINTS = (
     "hc_correlate1d",
     "hc_correlate_nd",
     "hc_separable2d",
+    "hc_separable2d_slices",
     "hc_hessian_gaussian",
     "hc_sym_eigvals",
     "hc_frangi",
@@ -147,6 +148,7 @@ _SIGNATURES = {
     "hc_correlate_nd": ([_A, _A, _v, _P(ctypes.c_int64), _P(ctypes.c_int32),
                          _P(ctypes.c_int32), _i, _d, _v], _i),
     "hc_separable2d": ([_A, _A, _T, _T, _i, _i, _d, _v], _i),
+    "hc_separable2d_slices": ([_A, _A, _T, _T, _i, _i, _d, _v], _i),
     "hc_hessian_gaussian": ([_A, _A, _i, _T, _T, _i, _d, _i, _v, _v], _i),
     "hc_sym_eigvals": ([_A, _i, _A, _i, _i, _v], _i),
     "hc_frangi": ([_A, _A, _T, _T, _i, _d, _d, _d, _i, _i, _i, _d, _A, _i, _v, _v, _v], _i),

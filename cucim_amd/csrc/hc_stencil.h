@@ -81,11 +81,16 @@ __host__ __device__ constexpr int reg_strip_outputs(int K) {
 constexpr int kRegKs[] = {3, 5, 7, 9, 13, 17, 21, 25, 33};
 constexpr int kRegMaxK = 33;
 
-// Fused two-pass 2-D filter of a float32 image into a float32 output (the
-// register-blocked kernel).  Returns HC_OK, or -1 when the arguments are
+// Fused two-pass 2-D filter of a float32 image, or of every slice of a stack,
+// into a float32 output (the register-blocked kernel).  Returns HC_OK, or -1 when the arguments are
 // outside what this kernel handles (the caller then uses the general tile
 // kernel).
 int launch_sep2d_reg(const hc_array* in, const hc_array* out, const hc_taps* t0,
                      const hc_taps* t1, int mode0, int mode1, double cval, hipStream_t st);
+
+// correlate1d along an axis that is not the last, float32, at most kRegMaxK
+// taps.  Returns HC_OK, or -1 when the arguments are outside what it handles.
+int launch_axis_reg(const hc_array* in, const hc_array* out, const hc_taps* t, int axis, int mode,
+                    double cval, hipStream_t st);
 
 }  // namespace hc

@@ -779,6 +779,10 @@ int hc_correlate1d(const hc_array* in, const hc_array* out, const hc_taps* taps,
     if (!fits) return fail(HC_ERR_RESOURCE, "kernel too long for the LDS-tiled line kernels");
   }
   const bool tiled = algorithm != HC_ALGO_GATHER && contig && fits;
+  if (tiled) {
+    rc = launch_axis_reg(in, out, taps, axis, mode, cval, st);
+    if (rc != -1) return rc;
+  }
   if (tiled)
     return f64 ? launch_tiled_1d<double>(in, out, taps, axis, mode, cval, st)
                : launch_tiled_1d<float>(in, out, taps, axis, mode, cval, st);
@@ -816,6 +820,23 @@ int hc_separable2d(const hc_array* in, const hc_array* out, const hc_taps* taps0
   if (rc != -1) return rc;
   return taps0->w_f64 ? launch_sep2d<double>(in, out, taps0, taps1, mode0, mode1, cval, st)
                       : launch_sep2d<float>(in, out, taps0, taps1, mode0, mode1, cval, st);
+}
+
+int hc_separable2d_slices(const hc_array* in, const hc_array* out, const hc_taps* taps0,
+                          const hc_taps* taps1, int mode0, int mode1, double cval, void* stream) {
+  int rc = check_in_out(in, out);
+  if (rc != HC_OK) return rc;
+  if (in->ndim != 3) return fail(HC_ERR_VALUE, "hc_separable2d_slices needs a 3-D array");
+  if (!valid_mode(mode0) || !valid_mode(mode1))
+    return fail(HC_ERR_VALUE, "boundary mode not supported");
+  if (!taps0 || !taps1) return fail(HC_ERR_VALUE, "null taps");
+  if (taps0->K < 1 || taps1->K < 1) return fail(HC_ERR_VALUE, "incorrect filter size");
+  if (taps0->anchor < 0 || taps0->anchor >= taps0->K || taps1->anchor < 0 ||
+      taps1->anchor >= taps1->K)
+    return fail(HC_ERR_VALUE, "invalid origin");
+  rc = launch_sep2d_reg(in, out, taps0, taps1, mode0, mode1, cval, (hipStream_t)stream);
+  if (rc == -1) return fail(HC_ERR_RESOURCE, "not a float32 stack with kernels of at most 33 taps");
+  return rc;
 }
 
 }  // extern "C"

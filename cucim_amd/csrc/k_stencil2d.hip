@@ -18,6 +18,7 @@ struct Reg2dArgs {
   float* out;
   int64_t H, W;
   int64_t ntx, ntiles;
+  int64_t per_slice;  // tiles of one (H, W) slice of a stack
   int TX;
   int a0, a1;  // anchors of the vertical / horizontal kernel
   int mode0, mode1;
@@ -25,11 +26,17 @@ struct Reg2dArgs {
 };
 
 template <int K, int TY>
-__global__ __launch_bounds__(256) void k_sep2d_reg(const Reg2dArgs a, const RegTaps<K> t0,
+__global__ __launch_bounds__(256) void k_sep2d_reg(Reg2dArgs a, const RegTaps<K> t0,
                                                    const RegTaps<K> t1) {
   __shared__ __align__(16) float U[TY * kRegUStride];
-  const int64_t tile = xcd_swizzle(blockIdx.x, gridDim.x);
-  const int64_t ty = tile / a.ntx, tx = tile - ty * a.ntx;
+  int64_t tile = xcd_swizzle(blockIdx.x, gridDim.x);
+  if (a.per_slice < a.ntiles) {
+    const int64_t slice = (unsigned)tile / (unsigned)a.per_slice;
+    tile -= slice * a.per_slice;
+    a.in += slice * a.H * a.W;
+    a.out += slice * a.H * a.W;
+  }
+  const int64_t ty = (unsigned)tile / (unsigned)a.ntx, tx = tile - ty * a.ntx;
   const int64_t y0 = ty * TY, x0 = tx * a.TX;
   const int c = threadIdx.x;
   // staged column; -1: outside the image in constant mode (intermediate = cval)
@@ -66,9 +73,11 @@ __global__ __launch_bounds__(256) void k_sep2d_reg(const Reg2dArgs a, const RegT
     float r[kRegP];
     reg_hpass<K>(r, U + i * kRegUStride + o, t1);
     float* op = a.out + y * a.W + x;
-    if (x + kRegP <= a.W && ((uintptr_t)op & 15) == 0) {
-      // streaming stores: the output is not read again by this launch
-      typedef float f4v __attribute__((ext_vector_type(4)));
+    if (x + kRegP <= a.W) {
+      // streaming stores: the output is not read again by this launch; 16
+      // bytes at any element (odd widths: 13 taps over 4032 x 3021 42 us with
+      // single stores, 29 us so)
+      typedef float f4v __attribute__((ext_vector_type(4), aligned(4)));
       __builtin_nontemporal_store(f4v{r[0], r[1], r[2], r[3]}, reinterpret_cast<f4v*>(op));
       __builtin_nontemporal_store(f4v{r[4], r[5], r[6], r[7]}, reinterpret_cast<f4v*>(op) + 1);
     } else {
@@ -88,14 +97,16 @@ void fill_taps(RegTaps<K>* r, const hc_taps* t) {
 }
 
 template <int K, int TY>
-int launch_reg(Reg2dArgs a, const hc_taps* t0, const hc_taps* t1, hipStream_t st) {
+int launch_reg(Reg2dArgs a, int64_t slices, const hc_taps* t0, const hc_taps* t1,
+               hipStream_t st) {
   RegTaps<K> r0, r1;
   fill_taps<K>(&r0, t0);
   fill_taps<K>(&r1, t1);
   a.TX = reg_strip_outputs(K);
   a.ntx = (a.W + a.TX - 1) / a.TX;
   const int64_t nty = (a.H + TY - 1) / TY;
-  a.ntiles = a.ntx * nty;
+  a.per_slice = a.ntx * nty;
+  a.ntiles = a.per_slice * slices;
   if (a.ntiles > 0x7fffffff) return fail(HC_ERR_VALUE, "array too large");
   HC_LAUNCH("k_sep2d_reg", st, (k_sep2d_reg<K, TY>), dim3((unsigned)a.ntiles), dim3(256), 0,
             a, r0, r1);
@@ -103,14 +114,15 @@ int launch_reg(Reg2dArgs a, const hc_taps* t0, const hc_taps* t1, hipStream_t st
 }
 
 template <int K>
-int launch_reg_ty(const Reg2dArgs& a, const hc_taps* t0, const hc_taps* t1, hipStream_t st) {
+int launch_reg_ty(const Reg2dArgs& a, int64_t slices, const hc_taps* t0, const hc_taps* t1,
+                  hipStream_t st) {
   // Default: 8 rows up to 4 Mpixel (2048^2: more work-groups for a launch
   // that is one wave of the chip, 18 vs 19 us), 16 above (8, 16 and 32 rows
   // measure within noise of each other at 8192^2)
   int ty = tune_get(HC_TUNE_SEP2D_TY);
-  if (ty != 8 && ty != 16 && ty != 32) ty = a.H * a.W <= (int64_t(1) << 22) ? 8 : 16;
-  if (ty == 8) return launch_reg<K, 8>(a, t0, t1, st);
-  return ty == 32 ? launch_reg<K, 32>(a, t0, t1, st) : launch_reg<K, 16>(a, t0, t1, st);
+  if (ty != 8 && ty != 16 && ty != 32) ty = slices * a.H * a.W <= (int64_t(1) << 22) ? 8 : 16;
+  if (ty == 8) return launch_reg<K, 8>(a, slices, t0, t1, st);
+  return ty == 32 ? launch_reg<K, 32>(a, slices, t0, t1, st) : launch_reg<K, 16>(a, slices, t0, t1, st);
 }
 
 }  // namespace
@@ -118,30 +130,135 @@ int launch_reg_ty(const Reg2dArgs& a, const hc_taps* t0, const hc_taps* t1, hipS
 int launch_sep2d_reg(const hc_array* in, const hc_array* out, const hc_taps* t0,
                      const hc_taps* t1, int mode0, int mode1, double cval, hipStream_t st) {
   if (in->dtype != HC_FLOAT32 || out->dtype != HC_FLOAT32 || t0->w_f64 || t1->w_f64) return -1;
-  if (!is_c_contiguous(in) || !is_c_contiguous(out) || in->ndim != 2) return -1;
+  if (!is_c_contiguous(in) || !is_c_contiguous(out) || in->ndim < 2 || in->ndim > 3) return -1;
+  const int d0 = in->ndim - 2;
+  const int64_t slices = d0 ? in->shape[0] : 1;
   const int64_t K = t0->K > t1->K ? t0->K : t1->K;
   if (K > kRegMaxK) return -1;
   Reg2dArgs a;
   std::memset(&a, 0, sizeof(a));
   a.in = (const float*)in->data;
   a.out = (float*)out->data;
-  a.H = in->shape[0];
-  a.W = in->shape[1];
+  a.H = in->shape[d0];
+  a.W = in->shape[d0 + 1];
   a.a0 = t0->anchor;
   a.a1 = t1->anchor;
   a.mode0 = mode0;
   a.mode1 = mode1;
   a.cval = (float)cval;
-  if (a.H == 0 || a.W == 0) return HC_OK;
-  if (K <= 3) return launch_reg_ty<3>(a, t0, t1, st);
-  if (K <= 5) return launch_reg_ty<5>(a, t0, t1, st);
-  if (K <= 7) return launch_reg_ty<7>(a, t0, t1, st);
-  if (K <= 9) return launch_reg_ty<9>(a, t0, t1, st);
-  if (K <= 13) return launch_reg_ty<13>(a, t0, t1, st);
-  if (K <= 17) return launch_reg_ty<17>(a, t0, t1, st);
-  if (K <= 21) return launch_reg_ty<21>(a, t0, t1, st);
-  if (K <= 25) return launch_reg_ty<25>(a, t0, t1, st);
-  return launch_reg_ty<33>(a, t0, t1, st);
+  if (slices == 0 || a.H == 0 || a.W == 0) return HC_OK;
+  if (K <= 3) return launch_reg_ty<3>(a, slices, t0, t1, st);
+  if (K <= 5) return launch_reg_ty<5>(a, slices, t0, t1, st);
+  if (K <= 7) return launch_reg_ty<7>(a, slices, t0, t1, st);
+  if (K <= 9) return launch_reg_ty<9>(a, slices, t0, t1, st);
+  if (K <= 13) return launch_reg_ty<13>(a, slices, t0, t1, st);
+  if (K <= 17) return launch_reg_ty<17>(a, slices, t0, t1, st);
+  if (K <= 21) return launch_reg_ty<21>(a, slices, t0, t1, st);
+  if (K <= 25) return launch_reg_ty<25>(a, slices, t0, t1, st);
+  return launch_reg_ty<33>(a, slices, t0, t1, st);
+}
+
+// ------------------------------------------------------ strided axis --
+// correlate1d of a float32 array along an axis that is not the last: a lane
+// owns one column (a line along the axis; neighbouring lanes neighbouring
+// columns of the flattened (outer, inner) index), loads the TY + K - 1 values
+// of TY outputs into registers, all before the first product, and applies the
+// taps as the fused filter's vertical pass does (the same bits as the LDS line
+// kernel).  Tiles of one column strip are consecutive, so the K - 1 rows two
+// of them share are read once from memory and once from the XCD's L2.  Bound
+// by memory.  13 taps over 201 x 387 x 413: 142 us with the LDS line kernel's
+// element-wise loads, 70 us here.
+namespace {
+
+struct AxisRegArgs {
+  const float* in;
+  float* out;
+  int64_t N, inner, ncols;  // axis length, its stride, number of lines
+  int64_t nty;              // tiles along the axis
+  int a0, mode;
+  float cval;
+};
+
+template <int K, int TY>
+__global__ __launch_bounds__(256) void k_axis_reg(const AxisRegArgs a, const RegTaps<K> t) {
+  const unsigned tile = (unsigned)xcd_swizzle(blockIdx.x, gridDim.x);
+  const unsigned strip = tile / (unsigned)a.nty;
+  const int64_t y0 = (int64_t)(tile - strip * (unsigned)a.nty) * TY, ya = y0 - a.a0;
+  const int64_t c = (int64_t)strip * 256 + threadIdx.x;
+  const int64_t cc = c < a.ncols ? c : a.ncols - 1;  // in bounds; not stored
+  const int64_t o = a.inner == a.ncols ? 0 : cc / a.inner;
+  const int64_t base = o * a.N * a.inner + (cc - o * a.inner);
+  float v[TY + K - 1];
+  if (ya >= 0 && ya + TY + K - 1 <= a.N) {
+    const float* col = a.in + base + ya * a.inner;
+#pragma unroll
+    for (int j = 0; j < TY + K - 1; ++j) v[j] = col[(int64_t)j * a.inner];
+  } else {
+#pragma unroll
+    for (int j = 0; j < TY + K - 1; ++j) {
+      const int64_t yr = remap(ya + j, a.N, a.mode);
+      v[j] = a.in[base + (yr >= 0 ? yr : 0) * a.inner];
+      if (yr < 0) v[j] = a.cval;
+    }
+  }
+  float acc[TY];
+  reg_vpass<K, TY>(acc, v, t);
+  if (c >= a.ncols) return;
+  float* op = a.out + base + y0 * a.inner;
+#pragma unroll
+  for (int i = 0; i < TY; ++i)
+    if (y0 + i < a.N) op[(int64_t)i * a.inner] = acc[i];
+}
+
+template <int K>
+int launch_axis_k(AxisRegArgs a, const hc_taps* t, hipStream_t st) {
+  RegTaps<K> r;
+  fill_taps<K>(&r, t);
+  const int64_t strips = (a.ncols + 255) / 256;
+  // 32 rows re-read (K - 1) / 32 of the input; fewer where that leaves CUs idle
+  const bool tall = strips * ((a.N + 31) / 32) >= 256 * 8;
+  a.nty = tall ? (a.N + 31) / 32 : (a.N + 7) / 8;
+  if (strips * a.nty > 0x7fffffff) return -1;
+  const dim3 g((unsigned)(strips * a.nty));
+  if (tall)
+    HC_LAUNCH("k_axis_reg", st, (k_axis_reg<K, 32>), g, dim3(256), 0, a, r);
+  else
+    HC_LAUNCH("k_axis_reg", st, (k_axis_reg<K, 8>), g, dim3(256), 0, a, r);
+  return HC_OK;
+}
+
+}  // namespace
+
+int launch_axis_reg(const hc_array* in, const hc_array* out, const hc_taps* t, int axis, int mode,
+                    double cval, hipStream_t st) {
+  if (in->dtype != HC_FLOAT32 || out->dtype != HC_FLOAT32 || t->w_f64 || t->K > kRegMaxK)
+    return -1;
+  if (!is_c_contiguous(in) || !is_c_contiguous(out)) return -1;
+  const Lines ln = lines_of(in, axis);
+  // The LDS line kernel's wide loads need rows that are whole 16-byte words:
+  // with them it is the faster one (8192^2, 17 taps: 113 us); without them, or
+  // where a wave's columns would span many rows, or in small arrays (8 to 10 us
+  // either way), the other way round (3000 x 4001, 17 taps: 48 us against 27).
+  const bool wide = ln.inner % 4 == 0 &&
+                    (((uintptr_t)in->data | (uintptr_t)out->data) & 15) == 0;
+  if (wide || ln.inner < 32 || numel(in) < (int64_t)1 << 20) return -1;
+  AxisRegArgs a;
+  std::memset(&a, 0, sizeof(a));
+  a.in = (const float*)in->data;
+  a.out = (float*)out->data;
+  a.N = ln.N;
+  a.inner = ln.inner;
+  a.ncols = ln.outer * ln.inner;
+  a.a0 = t->anchor;
+  a.mode = mode;
+  a.cval = (float)cval;
+  if (a.N == 0 || a.ncols == 0) return HC_OK;
+  if (t->K <= 3) return launch_axis_k<3>(a, t, st);
+  if (t->K <= 7) return launch_axis_k<7>(a, t, st);
+  if (t->K <= 13) return launch_axis_k<13>(a, t, st);
+  if (t->K <= 17) return launch_axis_k<17>(a, t, st);
+  if (t->K <= 25) return launch_axis_k<25>(a, t, st);
+  return launch_axis_k<33>(a, t, st);
 }
 
 // ------------------------------------------------------------------------

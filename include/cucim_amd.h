@@ -180,6 +180,11 @@ int hc_correlate_nd(const hc_array* in, const hc_array* out, const void* w_dev,
 int hc_separable2d(const hc_array* in, const hc_array* out, const hc_taps* taps0,
                    const hc_taps* taps1, int mode0, int mode1, double cval,
                    void* stream);
+/* the same over the last two axes of a C-contiguous float32 (slices, H, W)
+ * array in one launch; HC_ERR_RESOURCE for other dtypes or kernels of more
+ * than 33 taps */
+int hc_separable2d_slices(const hc_array* in, const hc_array* out, const hc_taps* taps0,
+                          const hc_taps* taps1, int mode0, int mode1, double cval, void* stream);
 
 /* Hessian by Gaussian derivatives for 2-D / 3-D float32/float64 images:
  * feature/corner.py:161-254 (_hessian_matrix_with_gaussian).

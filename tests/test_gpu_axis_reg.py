@@ -1,0 +1,73 @@
+"""The register line kernel of strided axes, the fused filter over stacks and
+the vector conversions: bit for bit what the element-wise kernel and the
+separate passes give, at tile edges, odd strides, unaligned arrays and with
+non-finite values."""
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _view(shape, off, seed, special=False):
+    """A float32 tensor that starts `off` elements into its storage."""
+    g = torch.Generator().manual_seed(seed)
+    n = int(np.prod(shape))
+    t = torch.randn(n + off, generator=g)
+    if special and n > 40:
+        t[off + n // 2] = float("inf")
+        t[off + n // 3] = float("nan")
+    return t.cuda()[off:].view(shape)
+
+
+@pytest.mark.parametrize("shape,axis", [((7, 32), 0), ((33, 257), 0), ((300, 513), 0),
+                                        ((2, 40, 33), 1), ((5, 9, 70), 0), ((3, 640, 655), 1),
+                                        ((1, 1, 40), 0), ((600, 4099), 0), ((1030, 1021), 0),
+                                        ((2, 3, 17, 45), 2)])
+@pytest.mark.parametrize("K,origin", [(1, 0), (3, 1), (4, 0), (8, -2), (13, 0), (18, 3), (33, 0)])
+@pytest.mark.parametrize("mode", ["reflect", "mirror", "nearest", "wrap", "constant"])
+def test_strided_axis_equals_gather(gpu, shape, axis, K, origin, mode):
+    from cucim_amd.skimage._vendored import ndimage as ndi
+
+    x = _view(shape, K % 2, K * 7 + axis, special=True)
+    w = np.random.default_rng(K).standard_normal(K).astype(np.float32)
+    if K > 4:
+        w[1] = 0  # a zero tap is skipped, also on inf and NaN
+    kw = dict(axis=axis, mode=mode, cval=1.5, origin=origin)
+    a = ndi.correlate1d(x, w, **kw)
+    b = ndi.correlate1d(x, w, algorithm="elementwise", **kw)
+    assert torch.equal(a.view(torch.int32)[~b.isnan()], b.view(torch.int32)[~b.isnan()])
+    assert torch.equal(a.isnan(), b.isnan())
+
+
+@pytest.mark.parametrize("shape", [(1, 5, 9), (3, 33, 240), (4, 17, 515), (2, 1, 300)])
+@pytest.mark.parametrize("sigma", [0.6, 1.5, (1.0, 2.0, 4.0), (0, 1.5, 2.0)])
+@pytest.mark.parametrize("mode", ["nearest", "reflect", "constant"])
+def test_stack_gaussian_equals_passes(gpu, monkeypatch, shape, sigma, mode):
+    from cucim_amd.skimage._vendored import _ndimage_filters as F
+
+    x = _view(shape, 1, 5)
+    a = F.gaussian_filter(x, sigma, mode=mode, cval=0.5)
+    y = x.clone()
+    F.gaussian_filter(y, sigma, mode=mode, cval=0.5, output=y)  # in place
+    t = torch.empty(shape[::-1], device="cuda").permute(2, 1, 0)
+    F.gaussian_filter(x.transpose(1, 2).contiguous().transpose(1, 2), sigma, mode=mode, cval=0.5,
+                      output=t)
+    monkeypatch.setattr(F, "FUSED_2D", False)
+    b = F.gaussian_filter(x, sigma, mode=mode, cval=0.5)
+    for got in (a, y, t):
+        assert torch.equal(got, b)
+
+
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 2047, 100003])
+@pytest.mark.parametrize("off", [0, 1, 3])
+def test_unsigned_to_float(gpu, n, off):
+    from cucim_amd.skimage.util import img_as_float32
+
+    rng = np.random.default_rng(n)
+    for dt, top in ((np.uint8, 255), (np.uint16, 65535)):
+        x = rng.integers(0, top + 1, n + off).astype(dt)
+        got = img_as_float32(torch.from_numpy(x).cuda()[off:]).cpu().numpy()
+        exp = x[off:].astype(np.float32) * np.float32(1.0 / top)
+        np.testing.assert_array_equal(got, exp)
