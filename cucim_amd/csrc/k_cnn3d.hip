@@ -15,8 +15,10 @@
 //       all on v_mfma_f32_16x16x32_bf16: lane l holds A[l % 16][8 (l / 16) + j],
 //       B[8 (l / 16) + j][l % 16] and D[4 (l / 16) + r][l % 16].  The weights
 //       are the A operand, so a lane ends with four consecutive channels of
-//       one voxel and stores them as one word.  Weights arrive pre-packed in
-//       each kernel's A order (k_pack_weights).
+//       one voxel and stores them as one word.  The bias is added to the
+//       finished sum (as the accumulators' start it would cost the products'
+//       partial sums its bits).  Weights arrive pre-packed in each kernel's A
+//       order (k_pack_weights).
 //   k_pad_bf16        reflect / nearest / ... padding of a float32 volume into
 //                     the bfloat16 single-channel input of the first layer
 //   training kernels  (float32): GELU backward, input gradient (full
@@ -171,9 +173,9 @@ k_conv3d_24x24(const ConvArgs a) {
 #pragma unroll
     for (int m = 0; m < MR; m += 2) {
       const int64_t o = o0 + (int64_t)m * OW * kC;
-      if (in && gy + m < OH) store_gelu4(a, o + ol, acc[m][0]);
-      if (in && gy + m + 1 < OH) store_gelu4(a, o + OW * kC + ol, acc[m + 1][0]);
-      const f32x4 v = join_halves(acc[m][1], acc[m + 1][1]);
+      if (in && gy + m < OH) store_gelu4(a, o + ol, acc[m][0] + bias0);
+      if (in && gy + m + 1 < OH) store_gelu4(a, o + OW * kC + ol, acc[m + 1][0] + bias0);
+      const f32x4 v = join_halves(acc[m][1], acc[m + 1][1]) + bias1;
       if (in && gy + m + k < OH) store_gelu4(a, o + k * OW * kC + oh, v);
     }
   };
@@ -194,7 +196,7 @@ k_conv3d_24x24(const ConvArgs a) {
     __syncthreads();
     if (late && prev >= 0) activate(prev);
 #pragma unroll
-    for (int m = 0; m < MR; ++m) acc[m][0] = bias0, acc[m][1] = bias1;
+    for (int m = 0; m < MR; ++m) acc[m][0] = acc[m][1] = f32x4{0.f, 0.f, 0.f, 0.f};
     const bf16x8* row = T + (pz * kTY + py) * k24Row + li * 3;
     // Pipelined by hand (left alone, the compiler reads a row right before its
     // products and waits for it): row i + 3 and one of the next step's weights
@@ -230,9 +232,12 @@ k_conv3d_24x24(const ConvArgs a) {
 
 // 1 -> 24.  The tile holds, per voxel, its value and the next two along x (and
 // a zero) as one 8-byte word: a lane's 8 values of K are two (dz, dy) rows of
-// three dx, so 9 rows make two steps.  Bound by the activation and the
-// stores: 8 waves of 8 rows, several work-groups per CU (0.69 ms of 264^3
-// voxels with a 2-byte LDS read per K value and a byte-wise store, 0.31 now).
+// three dx, and the ninth row's values take the free fourth places of the
+// first three lane groups, so one step holds all 27 taps (with a second step
+// for the ninth row the float32 sums were rounded once more).  Bound by the
+// activation and the stores: 8 waves of 8 rows, several work-groups per CU
+// (0.69 ms of 264^3 voxels with a 2-byte LDS read per K value and a byte-wise
+// store, 0.31 now).
 constexpr int k1BZ = 8;
 
 __global__ __launch_bounds__(64 * k1BZ) __attribute__((amdgpu_waves_per_eu(4))) void
@@ -243,21 +248,17 @@ k_conv3d_1x24(const ConvArgs a) {
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 15, kg = lane >> 4;
   const int OD = a.D - 2, OH = a.H - 2, OW = a.W - 2;
-  bf16x8 w[2][2];
-#pragma unroll
-  for (int c = 0; c < 2; ++c)
-#pragma unroll
-    for (int t = 0; t < 2; ++t) w[c][t] = a.wpk[(c * 2 + t) * 64 + lane];
+  const bf16x8 w0 = a.wpk[lane], w1 = a.wpk[64 + lane];
   f32x4 bias0, bias1;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     bias0[r] = a.bias[4 * kg + r];
     bias1[r] = a.bias[16 + 4 * (kg & 1) + r];
   }
-  // rows 2 kg and 2 kg + 1 of (dz, dy) in step 0, row 8 (group 0) in step 1
+  // rows 2 kg and 2 kg + 1 of (dz, dy), and dx = kg of row 8 (kg < 3)
   const int g0 = 2 * kg, g1 = 2 * kg + 1;
   const int off0 = (g0 / 3 * kTY + g0 % 3) * kTX, off1 = (g1 / 3 * kTY + g1 % 3) * kTX;
-  constexpr int off8 = (2 * kTY + 2) * kTX;
+  const int off8 = (2 * kTY + 2) * kTX + (kg < 3 ? kg : 0);
   const int64_t G = gridDim.x;
   for (int64_t blk = xcd_swizzle(blockIdx.x, G); blk < a.nblocks; blk += G) {
     int x0, y0, z0;
@@ -285,19 +286,19 @@ k_conv3d_1x24(const ConvArgs a) {
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
         const bf16x4* p = row + (m + k) * kTX;
-        const bf16x4 u = p[off0], v = p[off1];
-        bf16x4 q = p[off8];
-        if (kg != 0) q = bf16x4{};  // no weight: not even inf * 0
+        bf16x4 u = p[off0];
+        const bf16x4 v = p[off1];
+        const __bf16 q = p[off8][0];
+        u[3] = kg < 3 ? q : (__bf16)0.0f;  // no weight: not even inf * 0
         const bf16x8 x = __builtin_shufflevector(u, v, 0, 1, 2, 3, 4, 5, 6, 7);
-        const bf16x8 y = __builtin_shufflevector(q, bf16x4{}, 0, 1, 2, 3, 4, 5, 6, 7);
-        acc[k][0] = mfma_bf16(w[1][0], y, mfma_bf16(w[0][0], x, bias0));
-        acc[k][1] = mfma_bf16(w[1][1], y, mfma_bf16(w[0][1], x, bias1));
+        acc[k][0] = mfma_bf16(w0, x, f32x4{0.f, 0.f, 0.f, 0.f});
+        acc[k][1] = mfma_bf16(w1, x, f32x4{0.f, 0.f, 0.f, 0.f});
       }
 #pragma unroll
       for (int k = 0; k < 2; ++k)
         if (in && y0 + m + k < OH)
-          store_gelu4(a, o0 + (int64_t)(m + k) * OW * kC + 4 * kg, acc[k][0]);
-      const f32x4 v = join_halves(acc[0][1], acc[1][1]);
+          store_gelu4(a, o0 + (int64_t)(m + k) * OW * kC + 4 * kg, acc[k][0] + bias0);
+      const f32x4 v = join_halves(acc[0][1], acc[1][1]) + bias1;
       const int k = kg >> 1;
       if (in && y0 + m + k < OH)
         store_gelu4(a, o0 + (int64_t)(m + k) * OW * kC + 16 + 4 * (kg & 1), v);
@@ -547,10 +548,12 @@ __global__ __launch_bounds__(256) void k_pack_weights(const float* __restrict__ 
         if (q < 27) tap = q / 9 * 9 + dy * 3 + q / 3 % 3;
         ci = q % 3 * 8 + j;
         co = 16 * t + row;
-      } else if (CI == 1 && CO == 24) {  // [step][tile][lane]
-        const int t = i / 64 % 2, g = 8 * (i / 128) + 2 * kg + j / 4;
-        if (g < 9 && j % 4 < 3) tap = g * 3 + j % 4;
-        co = 16 * t + row;
+      } else if (CI == 1 && CO == 24) {  // [tile][lane]
+        if (j % 4 < 3)
+          tap = (2 * kg + j / 4) * 3 + j % 4;
+        else if (j == 3 && kg < 3)
+          tap = 24 + kg;
+        co = 16 * (i / 64) + row;
       } else if (CI == 24 && CO == 1) {  // [step][lane], row = (dz, dy)
         const int q = 4 * (i / 64) + kg;
         if (q < 9 && row < 9) tap = row * 3 + q / 3;
@@ -621,7 +624,7 @@ extern "C" {
 int hc_cnn3d_packed_size(int ci, int co) {
   if (ci < 1 || co < 1) return -1;
   if (ci == 24 && co == 24) return k24Steps * 6 * 64 * 16;
-  if (ci == 1 && co == 24) return 4 * 64 * 16;
+  if (ci == 1 && co == 24) return 2 * 64 * 16;
   if (ci == 24 && co == 1) return 3 * 64 * 16;
   return ((27 * ci + 31) / 32) * ((co + 15) / 16) * 64 * 16;
 }

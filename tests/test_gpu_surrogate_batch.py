@@ -66,6 +66,30 @@ def test_batched_forward(gpu, ci, co, act, shape):
         assert torch.equal(out.cpu(), (pre.clamp(0, 1) if act == 2 else pre).cpu())
 
 
+@pytest.mark.parametrize("ci,co,act", [(24, 24, 1), (1, 24, 1), (24, 1, 0)])
+@pytest.mark.parametrize("shape", [(1, 5, 11, 19), (3, 29, 59, 117)])
+def test_bias_is_added_to_the_finished_sum(gpu, ci, co, act, shape):
+    """Products 1 and -1 of the first and the last tap cancel exactly, so a
+    bias of 2^-30 comes back whole; added before the products, 1 + 2^-30
+    would round it away."""
+    from cucim_amd import _array
+    from cucim_amd import _lib as L
+
+    lib, st = L.lib(), _array.stream()
+    x = torch.ones(shape + (ci,), dtype=torch.bfloat16, device="cuda")
+    w = torch.zeros((27, ci, co), device="cuda")
+    w[0, 0], w[26, ci - 1] = 1, -1
+    b = 2.0 ** -30 * torch.arange(1, co + 1, device="cuda")
+    oshape = (shape[0],) + tuple(s - 2 for s in shape[1:]) + (co,)
+    out = torch.empty(oshape, dtype=torch.bfloat16 if co == 24 else torch.float32, device="cuda")
+    pre = torch.empty(oshape, device="cuda")
+    packed = torch.empty(lib.hc_cnn3d_packed_size(ci, co), dtype=torch.uint8, device="cuda")
+    L.check(lib.hc_cnn3d_pack(w.data_ptr(), packed.data_ptr(), ci, co, st))
+    L.check(lib.hc_cnn3d_conv(_array.hc_array(x), _array.hc_array(out), packed.data_ptr(),
+                              b.data_ptr(), act, pre.data_ptr(), st))
+    assert torch.equal(pre, b.expand(oshape))
+
+
 @pytest.mark.parametrize("ci,co", [(24, 24), (1, 24), (24, 1)])
 @pytest.mark.parametrize("shape", [(1, 3, 3, 3), (2, 4, 10, 18), (3, 5, 11, 19), (1, 20, 3, 35),
                                    (2, 13, 27, 9)])
