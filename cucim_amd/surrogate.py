@@ -229,23 +229,35 @@ class FrangiSurrogate:
 _BATCH_VOXELS = 8 * 64 ** 3
 
 
+def _target(x, t):
+    """The target of the patch ``x`` as a dense float32 array of its valid
+    outputs (the kernels read it by address)."""
+    shape = tuple(int(s) - 2 * HALO for s in x.shape[:3])
+    if not x.is_cuda or t.device != x.device:
+        raise ValueError("patches and targets must be on one GPU")
+    if t.dtype != torch.float32:
+        raise ValueError(f"targets must be float32, not {t.dtype}")
+    if t.numel() != math.prod(shape):
+        raise ValueError(f"a patch of shape {tuple(x.shape)} needs a target of shape {shape}, "
+                         f"not {tuple(t.shape)}")
+    return t.contiguous().view(shape)
+
+
 def _batches(xs, ts):
     """Consecutive patches of one shape stacked along a new first dimension,
     at most _BATCH_VOXELS input voxels (at least one patch) each.  A patch
-    whose input or target is not a dense array of the expected shape goes
-    alone."""
-    def shape_of(x, t):
-        ok = (x.dim() == 4 and x.is_contiguous() and t.dtype == torch.float32
-              and tuple(t.shape) == tuple(s - 2 * HALO for s in x.shape[:3]))
-        return (tuple(x.shape), x.dtype, x.device, t.device) if ok else None
+    that is not a dense (D, H, W, 1) array goes alone (and is refused by the
+    layers)."""
+    def shape_of(x):
+        return (tuple(x.shape), x.dtype, x.device) if x.dim() == 4 and x.is_contiguous() else None
 
-    pairs = list(zip(xs, ts))
+    pairs = [(x, _target(x, t)) for x, t in zip(xs, ts)]
     i = 0
     while i < len(pairs):
-        shape = shape_of(*pairs[i])
+        shape = shape_of(pairs[i][0])
         most = 1 if shape is None else max(1, _BATCH_VOXELS // pairs[i][0].numel())
         j = i + 1
-        while j < len(pairs) and j - i < most and shape_of(*pairs[j]) == shape:
+        while j < len(pairs) and j - i < most and shape_of(pairs[j][0]) == shape:
             j += 1
         if j - i == 1:
             yield pairs[i][0][None], pairs[i][1][None]

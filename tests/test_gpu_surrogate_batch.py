@@ -174,3 +174,43 @@ def test_step_batches_like_single_patches(gpu, monkeypatch):
     for a, b in zip(got[0][1], got[1][1]):
         assert float((a - b).norm()) <= 1e-5 * float(b.norm())
     assert np.isfinite(got[0][0])
+
+
+def _step(S, xs, ts):
+    m = S.FrangiSurrogate(seed=3)
+    loss = m.train_step(xs, ts)
+    return float(loss), [t.clone() for t in m._gw + m._gb]
+
+
+def test_targets_that_are_not_dense(gpu):
+    """A crop of a larger label volume, alone and among patches of its shape,
+    gives what its dense copy gives; so does a target with a channel axis."""
+    from cucim_amd import surrogate as S
+
+    g = torch.Generator().manual_seed(9)
+    xs = [torch.rand((14, 13, 15, 1), generator=g).to(torch.bfloat16).cuda() for _ in range(3)]
+    labels = [torch.rand((14, 13, 15), generator=g).cuda() for _ in range(3)]
+    crops = [t[5:-5, 5:-5, 5:-5] for t in labels]
+    assert not any(t.is_contiguous() for t in crops)
+    for n in (1, 3):
+        exp = _step(S, xs[:n], [t.contiguous() for t in crops[:n]])
+        for ts in (crops, [t[..., None] for t in crops]):
+            got = _step(S, xs[:n], ts[:n])
+            # the loss is added by atomics, in any order
+            assert abs(got[0] - exp[0]) <= 1e-6 * exp[0]
+            assert all(torch.equal(a, b) for a, b in zip(got[1], exp[1]))
+
+
+def test_targets_that_do_not_fit_are_refused(gpu):
+    from cucim_amd import surrogate as S
+
+    x = torch.zeros((13, 13, 13, 1), dtype=torch.bfloat16, device="cuda")
+    t = torch.zeros((3, 3, 3), device="cuda")
+    m = S.FrangiSurrogate(seed=3)
+    before = [w.clone() for w in m.w]
+    for bad in (t.double(), t.to(torch.bfloat16), t[:2], torch.zeros((4, 3, 3), device="cuda"),
+                t.cpu()):
+        for xs, ts in (([x], [bad]), ([x, x], [t, bad])):
+            with pytest.raises(ValueError):
+                m.train_step(xs, ts)
+    assert all(torch.equal(a, b) for a, b in zip(before, m.w))
