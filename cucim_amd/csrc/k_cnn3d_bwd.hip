@@ -6,7 +6,8 @@
 // D[4 (l / 16) + r][l % 16].  Every sum over voxels or channels is a float32
 // sum of exact products of float32 values (a bfloat16 activation widens
 // exactly), as in the per-output kernels these replace; only the order of the
-// terms differs.
+// terms differs.  No operand that pads a block is multiplied by one that may be
+// infinite or NaN: sums hold their own terms only, with such values too.
 //
 // One training step of eight 64^3 patches took 269 ms with one work-item per
 // output and one launch per patch (weight gradients 40 launches of 3.4 ms,
@@ -141,24 +142,32 @@ k_conv3d_wgrad_mfma(const BwdArgs a) {
     for (int u = 0; u < NG; ++u) reinterpret_cast<f32x4*>(G)[tid + 256 * u] = pg[u];
     if (blk + NB < a.nblocks) fetch(blk + NB);  // in flight during the products
     __syncthreads();
+    // outputs past the patch take no part: their rows and steps are left out,
+    // and in a row's last step the activations next to them are zeroed (only
+    // the gradient's tile is padded; 0 * inf would spoil a sum)
+    const Origin o = origin_of(a, blk);
+    const int nz = min(kBZ, OD - o.z), ny = min(kBY, OH - o.y), nx = min(kBX, OW - o.x);
 #pragma unroll 1
-    for (int r = 0; r < kBZ * kBY; ++r) {
+    for (int r = 0; r < nz * kBY; ++r) {
       const int z = r / kBY, y = r - z * kBY;
+      if (y >= ny) continue;
       const __bf16* xr = X + ((z * kTY + y) * kTX + kg) * kC;
       const float* gr = G + (r * kBX + kg) * kC + li;
-#pragma unroll 2
-      for (int s = 0; s < kBX / 4; ++s) {
+      auto step = [&](int s, bool in) {
         const float a0 = gr[4 * s * kC], a1 = gr[4 * s * kC + 16];
         float b[kWgT];
 #pragma unroll
-        for (int j = 0; j < kWgT; ++j) b[j] = bf2f(xr[toff[j] + 4 * s * kC]);
+        for (int j = 0; j < kWgT; ++j) b[j] = in ? bf2f(xr[toff[j] + 4 * s * kC]) : 0.f;
         if (one) b[kWgT - 1] = 1.f;
 #pragma unroll
         for (int j = 0; j < kWgT; ++j) {
           acc[0][j] = mfma_f32(a0, b[j], acc[0][j]);
           acc[1][j] = mfma_f32(a1, b[j], acc[1][j]);
         }
-      }
+      };
+#pragma unroll 2
+      for (int s = 0; s < nx / 4; ++s) step(s, true);
+      if (nx % 4) step(nx / 4, kg < nx % 4);
     }
   }
   // rows 4 kg + r (+ 16), column 16 tile + li -> part[column][channel]
@@ -179,7 +188,10 @@ k_conv3d_wgrad_mfma(const BwdArgs a) {
 // M = the 24 channels (and, for 24 -> 1, a row of ones: its product with tap 0
 // is the sum of dy), N = the 27 taps (and, for 1 -> 24, a column of ones).
 // F is read straight from memory (each wave 4 rows of 16 voxels), S from LDS;
-// bound by reading F.
+// bound by reading F.  Where F is padded (1 -> 24), S is zeroed beside it; where
+// S is (24 -> 1, outputs off the patch), which positions are depends on the
+// tap, so a wave with an infinite or NaN activation takes its products tap by
+// tap with both operands zeroed.
 template <bool FIRST>
 __global__ __launch_bounds__(256) void k_conv3d_wgrad_1c(const BwdArgs a) {
   __shared__ float S[kTV];
@@ -209,6 +221,8 @@ __global__ __launch_bounds__(256) void k_conv3d_wgrad_1c(const BwdArgs a) {
     const Origin o = origin_of(a, blk);
     // this wave's F values: 4 rows x 4 steps x 2 channel tiles
     float f0[16], f1[16];
+    unsigned fin = 0;   // bit u: step u's position is in F
+    float chk = 0.f;    // stays 0 while every value is finite
 #pragma unroll
     for (int u = 0; u < 16; ++u) {
       const int r = 4 * wv + u / 4, z = o.z + r / kBY, y = o.y + r % kBY;
@@ -216,6 +230,7 @@ __global__ __launch_bounds__(256) void k_conv3d_wgrad_1c(const BwdArgs a) {
       const bool in = z < FD && y < FH && x < FW;
       const int64_t v = ((o.n * FD + z) * FH + y) * FW + x;
       f0[u] = f1[u] = 0.f;
+      fin |= (unsigned)in << u;
       if (in) {
         if (FIRST) {
           f0[u] = a.dy[v * kC + li];
@@ -225,6 +240,7 @@ __global__ __launch_bounds__(256) void k_conv3d_wgrad_1c(const BwdArgs a) {
           if (li < 8) f1[u] = bf2f(a.x[v * kC + 16 + li]);
         }
       }
+      if (!FIRST) chk = fmaf(f1[u], 0.f, fmaf(f0[u], 0.f, chk));
       if (rowone) f1[u] = 1.f;
     }
     __syncthreads();
@@ -241,11 +257,38 @@ __global__ __launch_bounds__(256) void k_conv3d_wgrad_1c(const BwdArgs a) {
       S[e] = v;
     }
     __syncthreads();
+    if (!FIRST && __any(!(chk == 0.f))) {
+#pragma unroll 1
+      for (int tap = 0; tap < 27; ++tap) {
+        const int dz = tap / 9, dy = tap / 3 % 3, dx = tap % 3;
+        const int off = ((2 - dz) * kTY + 2 - dy) * kTX + 2 - dx;
+        f32x4 t0{0.f, 0.f, 0.f, 0.f}, t1 = t0;
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+          const int r = 4 * wv + u / 4;
+          const int z = o.z + r / kBY - dz, y = o.y + r % kBY - dy;
+          const int x = o.x + 4 * (u % 4) + kg - dx;
+          const bool in = z >= 0 && y >= 0 && x >= 0 && z < OD && y < OH && x < OW;
+          const float b =
+              in ? S[(r / kBY * kTY + r % kBY) * kTX + 4 * (u % 4) + kg + off] : 0.f;
+          t0 = mfma_f32(in ? f0[u] : 0.f, b, t0);
+          t1 = mfma_f32(in ? f1[u] : 0.f, b, t1);
+        }
+        if (li == tap % 16) {
+          if (tap < 16)
+            acc[0][0] += t0, acc[1][0] += t1;
+          else
+            acc[0][1] += t0, acc[1][1] += t1;
+        }
+      }
+      continue;
+    }
 #pragma unroll
     for (int u = 0; u < 16; ++u) {
       const int r = 4 * wv + u / 4;
       const float* s = S + (r / kBY * kTY + r % kBY) * kTX + 4 * (u % 4) + kg;
-      const float b0 = s[toff[0]], b1 = colone ? 1.f : s[toff[1]];
+      const bool in = !FIRST || (fin >> u & 1);
+      const float b0 = in ? s[toff[0]] : 0.f, b1 = colone ? 1.f : in ? s[toff[1]] : 0.f;
       acc[0][0] = mfma_f32(f0[u], b0, acc[0][0]);
       acc[0][1] = mfma_f32(f0[u], b1, acc[0][1]);
       acc[1][0] = mfma_f32(f1[u], b0, acc[1][0]);
@@ -306,7 +349,8 @@ __global__ __launch_bounds__(1024) void k_sum_parts(const float* __restrict__ pa
 // 8-byte words per operand row; rows are 26 words apart, which spreads them
 // over the banks (24 would put every eighth row on the same ones).  Bound by
 // the matrix cores: 24 instructions of 32 cycles per wave and tap for 12
-// 8-byte words.
+// 8-byte words.  An infinite or NaN weight (times the zeros around the
+// gradient) sends a work-group to sums over its own terms, one per work-item.
 constexpr int kDgS = 26;
 constexpr int kDgLds = (kTV + 27 * kC) * kDgS * 4;
 
@@ -324,8 +368,13 @@ k_conv3d_dgrad_mfma(const BwdArgs a) {
     *reinterpret_cast<f32x2*>(row + 4 * v) = f32x2{x[0], x[1]};
     *reinterpret_cast<f32x2*>(row + 4 * v + 2) = f32x2{x[2], x[3]};
   };
-  for (int e = tid; e < 27 * kC * 6; e += 512)
-    put(Wl + e / 6 * kDgS, e % 6, reinterpret_cast<const f32x4*>(a.w)[e]);
+  float chk = 0.f;  // stays 0 while every weight is finite
+  for (int e = tid; e < 27 * kC * 6; e += 512) {
+    const f32x4 w = reinterpret_cast<const f32x4*>(a.w)[e];
+    chk = fmaf(w[3], 0.f, fmaf(w[2], 0.f, fmaf(w[1], 0.f, fmaf(w[0], 0.f, chk))));
+    put(Wl + e / 6 * kDgS, e % 6, w);
+  }
+  const bool wbad = __syncthreads_or(!(chk == 0.f));
   constexpr int NG = (kTV * 6 + 511) / 512;
   f32x4 pg[NG];
   auto fetch = [&](int64_t b) {
@@ -360,6 +409,27 @@ k_conv3d_dgrad_mfma(const BwdArgs a) {
     }
     if (blk + NB < a.nblocks) fetch(blk + NB);  // in flight during the products
     __syncthreads();
+    if (wbad) {  // uniform
+#pragma unroll 1
+      for (int e = tid; e < kBV * kC; e += 512) {
+        const int ci = e % kC, v = e / kC;
+        const int lx = v % kBX, ly = v / kBX % kBY, lz = v / (kBX * kBY);
+        const int gx = o.x + lx, gy = o.y + ly, gz = o.z + lz;
+        if (gx >= a.W || gy >= a.H || gz >= a.D) continue;
+        float s = 0.f;
+#pragma unroll 1
+        for (int tap = 0; tap < 27; ++tap) {
+          const int dz = tap / 9, dy = tap / 3 % 3, dx = tap % 3;
+          if (gz < dz || gy < dy || gx < dx || gz - dz >= OD || gy - dy >= OH || gx - dx >= OW)
+            continue;
+          const float* g = G + (((lz + 2 - dz) * kTY + ly + 2 - dy) * kTX + lx + 2 - dx) * kDgS;
+          for (int c = 0; c < kC; ++c) s = fmaf(g[c], Wl[(tap * kC + ci) * kDgS + c], s);
+        }
+        const int64_t q = (((o.n * a.D + gz) * a.H + gy) * a.W + gx) * kC + ci;
+        a.out[q] = a.pre ? s * gelu_grad(a.pre[q]) : s;
+      }
+      continue;
+    }
     f32x4 acc[2][2];
 #pragma unroll
     for (int m = 0; m < 2; ++m) acc[m][0] = acc[m][1] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -405,11 +475,15 @@ k_conv3d_dgrad_mfma(const BwdArgs a) {
 }
 
 // The same for 24 -> 1: one voxel per work-item, its 27 gradients from LDS,
-// 24 sums over the taps with wave-uniform weights.  Bound by writing dx.
+// 24 sums over the taps with wave-uniform weights (taps off the patch are left
+// out where a weight is not finite).  Bound by writing dx.
 __global__ __launch_bounds__(256) void k_conv3d_dgrad_1c(const BwdArgs a) {
   __shared__ float S[kTV];
   const int tid = threadIdx.x;
   const int OD = a.D - 2, OH = a.H - 2, OW = a.W - 2;
+  float chk = 0.f;  // stays 0 while every weight is finite
+  for (int e = tid; e < 27 * kC; e += 256) chk = fmaf(a.w[e], 0.f, chk);
+  const bool wbad = __syncthreads_or(!(chk == 0.f));
   for (int64_t blk = xcd_swizzle(blockIdx.x, gridDim.x); blk < a.nblocks; blk += gridDim.x) {
     const Origin o = origin_of(a, blk);
     __syncthreads();
@@ -424,16 +498,20 @@ __global__ __launch_bounds__(256) void k_conv3d_dgrad_1c(const BwdArgs a) {
     float acc[kC];
 #pragma unroll
     for (int c = 0; c < kC; ++c) acc[c] = 0.f;
+    const int px = o.x + lx, py = o.y + ly, pz = o.z + lz;
 #pragma unroll 3
     for (int tap = 0; tap < 27; ++tap) {
+      if (wbad) {
+        const int z = pz - tap / 9, y = py - tap / 3 % 3, x = px - tap % 3;
+        if (x < 0 || y < 0 || z < 0 || x >= OW || y >= OH || z >= OD) continue;
+      }
       const float g =
           S[((lz + 2 - tap / 9) * kTY + ly + 2 - tap / 3 % 3) * kTX + lx + 2 - tap % 3];
 #pragma unroll
       for (int c = 0; c < kC; ++c) acc[c] = fmaf(g, a.w[tap * kC + c], acc[c]);
     }
-    const int gx = o.x + lx, gy = o.y + ly, gz = o.z + lz;
-    if (gx < a.W && gy < a.H && gz < a.D) {
-      const int64_t q = (((o.n * a.D + gz) * a.H + gy) * a.W + gx) * kC;
+    if (px < a.W && py < a.H && pz < a.D) {
+      const int64_t q = (((o.n * a.D + pz) * a.H + py) * a.W + px) * kC;
 #pragma unroll
       for (int v = 0; v < kC / 4; ++v) {
         f32x4 r{acc[4 * v], acc[4 * v + 1], acc[4 * v + 2], acc[4 * v + 3]};

@@ -140,6 +140,65 @@ def test_batched_gradients(gpu, ci, co, shape):
         assert bool((err <= (27 * co + 2) * EPS * m + slack).all())
 
 
+@pytest.mark.parametrize("ci,co", [(24, 24), (1, 24), (24, 1)])
+@pytest.mark.parametrize("shape", [(1, 3, 3, 3), (2, 4, 10, 18), (2, 5, 11, 21), (1, 20, 3, 35)])
+def test_gradients_of_infinite_values_hold_their_own_terms(gpu, ci, co, shape):
+    """An infinite activation, gradient or weight makes those sums infinite or
+    NaN that contain it, and no others (the blocks are padded with zeros).
+    The reference adds the same terms in float64, tap by tap."""
+    from cucim_amd import _array
+    from cucim_amd import _lib as L
+
+    lib, st = L.lib(), _array.stream()
+    B, D, H, W = shape
+    OD, OH, OW = D - 2, H - 2, W - 2
+    g = torch.Generator().manual_seed(11)
+    x0 = torch.randn(shape + (ci,), generator=g).to(torch.bfloat16)
+    w0 = torch.randn((27, ci, co), generator=g) / 25
+    dy0 = torch.randn((B, OD, OH, OW, co), generator=g)
+
+    def reference(x, w, dy):
+        dw, dx = torch.zeros_like(w), torch.zeros_like(x)
+        f = dy.reshape(-1, co)
+        for t in range(27):
+            cut = (slice(None), slice(t // 9, t // 9 + OD), slice(t // 3 % 3, t // 3 % 3 + OH),
+                   slice(t % 3, t % 3 + OW))
+            dw[t] = (x[cut].reshape(-1, ci)[:, :, None] * f[:, None, :]).sum(0)
+            dx[cut] += (dy[..., None, :] * w[t]).sum(-1)
+        return dw, f.sum(0), dx
+
+    mag = reference(x0.double().abs(), w0.double().abs(), dy0.double().abs())
+    work = torch.empty(lib.hc_cnn3d_wgrad_work(ci, co), device="cuda")
+    for where in ("x last", "x first", "dy", "w"):
+        x, w, dy = x0.clone(), w0.clone(), dy0.clone()
+        if where == "x last":
+            x[-1, -1, -1, -1, 0] = float("inf")
+        elif where == "x first":
+            x[0, 0, 0, 0, ci - 1] = float("nan")
+        elif where == "dy":
+            dy[0, OD - 1, OH // 2, OW - 1, co - 1] = -float("inf")
+        else:
+            w[13, ci - 1, 0] = float("inf")
+        dw_r, db_r, dx_r = reference(x.double(), w.double(), dy.double())
+        xd, wd, dyd = x.cuda(), w.cuda(), dy.cuda()
+        dw, db = torch.zeros((27, ci, co), device="cuda"), torch.zeros(co, device="cuda")
+        L.check(lib.hc_cnn3d_wgrad_batch(xd.data_ptr(), dyd.data_ptr(), dw.data_ptr(),
+                                         db.data_ptr(), B, D, H, W, ci, co, work.data_ptr(),
+                                         work.numel(), st))
+        terms = B * OD * OH * OW + 512
+        res = [(dw, dw_r, mag[0], terms), (db, db_r, mag[1], terms)]
+        if ci > 1:
+            dx = torch.empty(shape + (ci,), device="cuda")
+            L.check(lib.hc_cnn3d_dgrad_batch(dyd.data_ptr(), wd.data_ptr(), None, dx.data_ptr(),
+                                             B, D, H, W, ci, co, st))
+            res.append((dx, dx_r, mag[2], 27 * co + 2))
+        for got, ref, m, n in res:
+            got = got.double().cpu()
+            fin = ref.isfinite()
+            assert torch.equal(got[~fin].nan_to_num(7.0), ref[~fin].nan_to_num(7.0)), where
+            assert bool(((got[fin] - ref[fin]).abs() <= n * EPS * m[fin]).all()), where
+
+
 def test_wgrad_work_is_checked(gpu):
     from cucim_amd import _array
     from cucim_amd import _lib as L
