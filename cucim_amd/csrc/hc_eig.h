@@ -150,15 +150,22 @@ __device__ __forceinline__ void eig33(F aa, F bb, F cc, F dd, F ee, F ff, int de
   // cos((phi - pi) / 3) and cos((phi + pi) / 3)
   double x1_term, ct, st;
   if constexpr (sizeof(F) == 4) {
-    // cos(phi) = x2 / (2 x1^(3/2)); x1 of floats is 0 or at least 1e-91.  With
-    // x1 = 0 every x2 but NaN gives phi = pi / 2, as below.  An infinite x1
-    // (from infinite elements of opposite signs) gives NaN.
-    const double y = x1 > 1e-200 ? rsqrt_fast(x1) : 0.0;
-    x1_term = (2.0 / 3.0) * (x1 * y);
-    const double cp = x2 * (0.5 * y * y * y);
-    const double s2 = fmax(fma(-cp, cp, 1.0), 0.0);
-    const double sp = s2 > 1e-200 ? s2 * rsqrt_fast(s2) : 0.0;
-    third_angle(cp, sp, ct, st);
+    if (x1 < HUGE_VAL && fabs(x2) < HUGE_VAL) {
+      // cos(phi) = x2 / (2 x1^(3/2)); x1 of floats is 0 or at least 1e-91.
+      // With x1 = 0 the angle does not matter.
+      const double y = x1 > 1e-200 ? rsqrt_fast(x1) : 0.0;
+      x1_term = (2.0 / 3.0) * (x1 * y);
+      const double cp = x2 * (0.5 * y * y * y);
+      const double s2 = fmax(fma(-cp, cp, 1.0), 0.0);
+      const double sp = s2 > 1e-200 ? s2 * rsqrt_fast(s2) : 0.0;
+      third_angle(cp, sp, ct, st);
+    } else {
+      // an infinite or NaN element: the angles that the arctangent below
+      // gives there (x2 = +-inf: 0 or pi; x2 finite: pi / 2; NaN: NaN)
+      const double phi = x2 != x2 ? x2 : fabs(x2) < HUGE_VAL ? M_PI / 2.0 : x2 > 0 ? 0.0 : M_PI;
+      x1_term = x1 < HUGE_VAL ? (2.0 / 3.0) * sqrt(x1) : x1;
+      sincos_small(phi * third, ct, st);
+    }
   } else {
     double phi;
     if (x2 == 0.0) {

@@ -57,3 +57,58 @@ def test_eigenvalues_of_zero_and_nan(gpu):
     el[1][0, 0, 0] = float("nan")
     for v in hessian_matrix_eigvals(el):
         assert bool(v[0, 0, 0].isnan()) and int(v.isnan().sum()) == 1
+
+
+def _closed_form(a, b, c, d, e, f):
+    """The closed form in float64 of [[a, d, f], [d, b, e], [f, e, c]], its
+    results in float32 after the descending compare-swaps."""
+    with np.errstate(all="ignore"):
+        a, b, c, d, e, f = (np.float64(v) for v in (a, b, c, d, e, f))
+        ta, tb, tc = 2 * a - b - c, 2 * b - a - c, 2 * c - a - b
+        x2 = -ta * tb * tc + 9 * (tc * (d * d) + tb * (f * f) + ta * (e * e)) - 54 * (d * e * f)
+        x1 = (a * a + b * b + c * c - a * b - a * c - b * c
+              + 3 * (d * d + e * e + f * f))
+        x1 = np.fmax(x1, 0.0)
+        if x2 == 0:
+            phi = np.pi / 2
+        else:
+            phi = np.arctan(np.sqrt(np.fmax(4 * x1 ** 3 - x2 * x2, 0.0)) / x2)
+            if x2 < 0:
+                phi += np.pi
+        m, t = (a + b + c) / 3, 2 / 3 * np.sqrt(x1)
+        l1 = np.float32(m - t * np.cos(phi / 3))
+        l2 = np.float32(m + t * np.cos((phi - np.pi) / 3))
+        l3 = np.float32(m + t * np.cos((phi + np.pi) / 3))
+        v1, v2, v3 = l3, l2, l1
+        if v1 > v2:
+            v1, v2 = v2, v1
+        if v1 > v3:
+            v1, v3 = v3, v1
+        if v2 > v3:
+            v2, v3 = v3, v2
+        return v3, v2, v1
+
+
+def test_eigenvalues_with_infinite_elements(gpu):
+    """One element infinite, of either sign, in any place: what the closed
+    form with a double arctangent gives, infinities and NaN alike."""
+    from cucim_amd.skimage.feature import hessian_matrix_eigvals
+
+    cases = []
+    for base in ((1, 2, 3, 0.5, -0.1, 0.1), (0, 0, 0, 0, 0, 0), (1, 2, 3, 0, 0, 0),
+                 (-1, 4, -2, 0.3, 0, 0.7)):
+        for k in range(6):
+            for v in (float("inf"), -float("inf")):
+                m = list(base)
+                m[k] = v
+                cases.append(m)
+    m = np.array(cases, np.float32)
+    assert m.shape == (48, 6)
+    el = [torch.from_numpy(np.ascontiguousarray(m[:, i])).cuda().view(2, 4, 6)
+          for i in (0, 3, 5, 1, 4, 2)]  # 00 01 02 11 12 22
+    got = torch.stack(list(hessian_matrix_eigvals(el))).cpu().numpy().reshape(3, -1).T
+    exp = np.array([_closed_form(*r) for r in m], np.float32)
+    exp.sort(axis=1)
+    got = np.sort(got, axis=1)
+    np.testing.assert_array_equal(got, exp)
+    assert np.isinf(exp).any() and np.isnan(exp).any()
