@@ -84,18 +84,22 @@ __device__ __forceinline__ double rsqrt_fast(double x) {
   return fma(y * e, fma(e, 0.375, 0.5), y);
 }
 
-// cos(phi / 3) and sin(phi / 3) of the angle phi in [0, pi] with cosine c and
-// sine s (doubles): the angle in float, then one Newton step for w^3 = c + i s
-// on the unit circle, w1 = (2 w0 + z conj(w0)^2 / |w0|^4) / 3, whose error is
-// the square of w0's (3e-7 at most): 1e-13 against 1e-16 of a double arctangent
-// and its sine and cosine, which took twice the instructions; the float
-// rounding of the eigenvalues is 6e-8.  atan(t) on [0, 1] by the minimax-like
-// odd polynomial of Abramowitz & Stegun 4.4.49 (2e-8); the sine and cosine by
-// their Taylor series on [0, pi / 3].
+// cos(phi / 3) and sin(phi / 3) of the angle phi in [0, pi] of the point
+// (c, s) on the unit circle (to an ulp of double; both 0 give phi = 0): the
+// angle in float, then the rotation by a third of what w0^3 lacks of it.  With
+// w0 = c0 + i s0 within 3e-7 of the result, m = |w0|^2 - 1 and
+// d = Im((c + i s) conj(w0)^3), the angle lacking is d (1 - 3 m / 2) (the terms
+// left out are below 1e-18), and w0 / |w0| turned by a third of it is
+// w0 (1 - m / 2 + 3 m^2 / 8 - t^2 / 2 + i t) with t = (1 - 2 m) d / 3.  As
+// accurate as a double arctangent with its sine and cosine (errors of the
+// eigenvalues against 80-bit ones the same to three digits, near equal
+// eigenvalues too) for half the instructions.  atan(t) on [0, 1] by the odd
+// polynomial of Abramowitz & Stegun 4.4.49 (2e-8); the sine and cosine by their
+// Taylor series on [0, pi / 3].
 __device__ __forceinline__ void third_angle(double c, double s, double& ct, double& st) {
   const float cf = (float)c, sf = (float)s, ca = fabsf(cf);
   const float hi = fmaxf(ca, sf), lo = fminf(ca, sf);
-  const float t = lo * __builtin_amdgcn_rcpf(hi), z = t * t;
+  const float a = lo * __builtin_amdgcn_rcpf(fmaxf(hi, 1e-30f)), z = a * a;
   float p = fmaf(z, 0.0028662257f, -0.0161657367f);
   p = fmaf(p, z, 0.0429096138f);
   p = fmaf(p, z, -0.0752896400f);
@@ -103,7 +107,7 @@ __device__ __forceinline__ void third_angle(double c, double s, double& ct, doub
   p = fmaf(p, z, -0.1420889944f);
   p = fmaf(p, z, 0.1999355085f);
   p = fmaf(p, z, -0.3333314528f);
-  float phi = fmaf(t * z, p, t);
+  float phi = fmaf(a * z, p, a);
   if (sf > ca) phi = 1.57079632679f - phi;
   if (cf < 0.f) phi = 3.14159265359f - phi;
   const float th = phi * 0.333333333f, q = th * th;
@@ -111,16 +115,20 @@ __device__ __forceinline__ void third_angle(double c, double s, double& ct, doub
   k = fmaf(k, q, -1.3888889e-3f);
   k = fmaf(k, q, 4.1666667e-2f);
   k = fmaf(k, q, -0.5f);
-  float m = fmaf(q, -2.5052108e-8f, 2.7557319e-6f);
-  m = fmaf(m, q, -1.9841270e-4f);
-  m = fmaf(m, q, 8.3333333e-3f);
-  m = fmaf(m, q, -0.16666667f);
-  const double c0 = (double)fmaf(k, q, 1.f), s0 = (double)fmaf(m * q, th, th);
-  const double cc = c0 * c0, ss = s0 * s0, f = fma(-2.0, cc + ss, 3.0);  // 1 / |w0|^4
-  const double u = f * (cc - ss), v = -2.0 * f * (c0 * s0);              // conj(w0)^2 / |w0|^4
+  float l = fmaf(q, -2.5052108e-8f, 2.7557319e-6f);
+  l = fmaf(l, q, -1.9841270e-4f);
+  l = fmaf(l, q, 8.3333333e-3f);
+  l = fmaf(l, q, -0.16666667f);
+  const double c0 = (double)fmaf(k, q, 1.f), s0 = (double)fmaf(l * q, th, th);
+  const double cs2 = 2.0 * (c0 * s0), w2 = fma(c0, c0, -s0 * s0);             // w0^2
+  const double w3r = fma(w2, c0, -cs2 * s0), w3i = fma(w2, s0, cs2 * c0);     // w0^3
+  const double m = fma(c0, c0, fma(s0, s0, -1.0));
   constexpr double third = 1.0 / 3.0;
-  ct = third * fma(2.0, c0, fma(c, u, -s * v));
-  st = third * fma(2.0, s0, fma(c, v, s * u));
+  const double d3 = third * fma(s, w3r, -c * w3i);
+  const double t = fma(-2.0 * m, d3, d3);
+  const double g = fma(m, fma(0.375, m, -0.5), -0.5 * t * t);
+  ct = c0 + fma(c0, g, -t * s0);
+  st = s0 + fma(s0, g, t * c0);
 }
 
 // 3x3, Deledalle et al. (2017) closed form in double (corner.py:566-612) for
@@ -151,14 +159,17 @@ __device__ __forceinline__ void eig33(F aa, F bb, F cc, F dd, F ee, F ff, int de
   double x1_term, ct, st;
   if constexpr (sizeof(F) == 4) {
     if (x1 < HUGE_VAL && fabs(x2) < HUGE_VAL) {
-      // cos(phi) = x2 / (2 x1^(3/2)); x1 of floats is 0 or at least 1e-91.
-      // With x1 = 0 the angle does not matter.
+      // cos(phi) = x2 / (2 x1^(3/2)), sin(phi) = sqrt(4 x1^3 - x2^2) / (2 x1^(3/2));
+      // the difference is taken before the scaling, as below: from cos(phi)
+      // rounded, it would be up to 1.7 times further off where two eigenvalues
+      // meet.  x1 of floats is 0 or at least 1e-91; with x1 = 0 the angle does
+      // not matter.
       const double y = x1 > 1e-200 ? rsqrt_fast(x1) : 0.0;
       x1_term = (2.0 / 3.0) * (x1 * y);
-      const double cp = x2 * (0.5 * y * y * y);
-      const double s2 = fmax(fma(-cp, cp, 1.0), 0.0);
-      const double sp = s2 > 1e-200 ? s2 * rsqrt_fast(s2) : 0.0;
-      third_angle(cp, sp, ct, st);
+      const double h = 0.5 * y * y * y;
+      const double arg = fmax(4 * x1 * x1 * x1 - x2 * x2, 0.0);
+      const double sp = arg > 0.0 ? arg * rsqrt_fast(arg) * h : 0.0;
+      third_angle(x2 * h, sp, ct, st);
     } else {
       // an infinite or NaN element: the angles that the arctangent below
       // gives there (x2 = +-inf: 0 or pi; x2 finite: pi / 2; NaN: NaN)

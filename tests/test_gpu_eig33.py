@@ -1,10 +1,10 @@
-"""Float32 3 x 3 eigenvalues (angle by float estimate and one Newton step)
+"""Float32 3 x 3 eigenvalues (the angle from a float estimate, corrected in double)
 against numpy in float64, over magnitudes from denormal cubes to 1e15 and the
 cases where two or three eigenvalues meet; and the float vesselness of the
 first sigma at small and large exponents.
 
 The result is rounded to float32 once (2^-24 of itself); the closed form in
-double adds 1e-13 of the largest eigenvalue, and sqrt(2^-52) = 1.5e-8 of it
+double adds 1e-16 of the largest eigenvalue, and sqrt(2^-52) = 1.5e-8 of it
 where two eigenvalues meet (the sine of the angle is the root of a rounded
 difference): 2^-23 of the largest eigenvalue bounds both."""
 
@@ -47,6 +47,40 @@ def test_eigenvalues_against_double(gpu, kind, scale):
     exp = np.linalg.eigvalsh(m.astype(np.float64))[:, ::-1].T
     top = np.abs(exp).max(0)
     assert (np.abs(got - exp) <= 2.0 ** -23 * top + 1e-44).all()
+
+
+def _eigenvalues(m, dtype):
+    """The closed form of symmetric float32 matrices in `dtype`, descending
+    and rounded to float32."""
+    a, d, f, b, e, c = (m[:, i, j].astype(dtype)
+                        for i, j in ((0, 0), (0, 1), (0, 2), (1, 1), (1, 2), (2, 2)))
+    ta, tb, tc = 2 * a - b - c, 2 * b - a - c, 2 * c - a - b
+    x2 = -ta * tb * tc + 9 * (tc * (d * d) + tb * (f * f) + ta * (e * e)) - 54 * (d * e * f)
+    x1 = a * a + b * b + c * c - a * b - a * c - b * c + 3 * (d * d + e * e + f * f)
+    th = np.arctan2(np.sqrt(np.maximum(4 * x1 * x1 * x1 - x2 * x2, 0)), x2) / 3
+    t, mid, third = 2 * np.sqrt(x1) / 3, (a + b + c) / 3, np.arccos(dtype(-1)) / 3
+    lam = np.stack([mid - t * np.cos(th), mid + t * np.cos(third - th),
+                    mid + t * np.cos(third + th)])
+    return np.sort(lam, axis=0)[::-1].astype(np.float32)
+
+
+def test_eigenvalues_of_equal_pairs_round_as_in_double(gpu):
+    """Where two eigenvalues meet, an error of the angle's sine, the root of a
+    rounded difference, moves some results to the next float: as many of them
+    as the closed form in double does (a tenth more for the order of its
+    roundings), against 80 bits.  A sine from the rounded cosine moves half as
+    many again."""
+    from cucim_amd.skimage.feature import hessian_matrix_eigvals
+
+    if np.finfo(np.longdouble).nmant < 63:
+        pytest.skip("needs 80-bit long double")
+    m = _matrices("pair", 60000, np.random.default_rng(8)).astype(np.float32)
+    el = [torch.from_numpy(np.ascontiguousarray(m[:, i, j])).cuda().view(30, 40, 50)
+          for i, j in ((0, 0), (0, 1), (0, 2), (1, 1), (1, 2), (2, 2))]
+    got = torch.stack(list(hessian_matrix_eigvals(el))).cpu().numpy().reshape(3, -1)
+    exact = _eigenvalues(m, np.longdouble)
+    moved = np.count_nonzero(_eigenvalues(m, np.float64) != exact)
+    assert 0 < np.count_nonzero(got != exact) <= 1.1 * moved
 
 
 def test_eigenvalues_of_zero_and_nan(gpu):
