@@ -1,7 +1,7 @@
 """Float32 3 x 3 eigenvalues (the angle from a float estimate, corrected in double)
 against numpy in float64, over magnitudes from denormal cubes to 1e15 and the
-cases where two or three eigenvalues meet; and the float vesselness of the
-first sigma at small and large exponents.
+cases where two or three eigenvalues meet; and the float32 vesselness's
+1 - e^x at exponents from 1e-16 to 200 and infinity.
 
 The result is rounded to float32 once (2^-24 of itself); the closed form in
 double adds 1e-16 of the largest eigenvalue, and sqrt(2^-52) = 1.5e-8 of it
@@ -146,3 +146,49 @@ def test_eigenvalues_with_infinite_elements(gpu):
     got = np.sort(got, axis=1)
     np.testing.assert_array_equal(got, exp)
     assert np.isinf(exp).any() and np.isnan(exp).any()
+
+
+def _gamma_factor(shape):
+    """An image whose midrange is 0 (nothing is subtracted before its Hessian),
+    its r_g, computed as the kernels do, and where the voxel's eigenvalues are
+    such that with alpha -> 0 and beta -> infinity the vesselness is exactly
+    its gamma factor 1 - e^(-r_g / 2 gamma^2)."""
+    from cucim_amd.skimage.feature import hessian_matrix, hessian_matrix_eigvals
+
+    x = np.random.default_rng(0).uniform(-0.9, 0.9, shape).astype(np.float32)
+    x.flat[0], x.flat[1] = -1, 1
+    xd = torch.from_numpy(x).cuda()
+    H = hessian_matrix(xd, sigma=1.5, mode="reflect", use_gaussian_derivatives=True)
+    l = torch.stack(list(hessian_matrix_eigvals(H))).cpu().numpy().reshape(len(shape), -1)
+    s = np.take_along_axis(l, np.argsort(np.abs(l), axis=0, kind="stable"), 0)
+    a = np.abs(s)
+    ok = (s[1:] > 1e-4).all(0) & (a[0] > 1e-6) & (a[1:] > 1.001 * a[:-1]).all(0)
+    rg = s[0] * s[0]
+    for v in s[1:]:  # fma
+        rg = (v.astype(np.longdouble) ** 2 + rg.astype(np.longdouble)).astype(np.float32)
+    assert np.count_nonzero(ok) > 10000
+    return xd, rg, ok
+
+
+def _ulps(got, exact):
+    return np.abs(got - exact) / np.spacing(exact.astype(np.float32)).astype(np.float64)
+
+
+@pytest.mark.parametrize("shape", [(48, 50, 52), (300, 310)])
+def test_vesselness_one_minus_exp(gpu, shape):
+    """expm1 in float: 0.89 ulp at most over all its arguments (measured), so
+    1 here."""
+    from cucim_amd.skimage.filters import frangi
+
+    x, rg, ok = _gamma_factor(shape)
+    top = float(np.sqrt(rg[ok].max()))
+    for g in (1e6 * top, 1e3 * top, 10 * top, top, top / 2, top / 4, top / 20):
+        out = frangi(x, sigmas=[1.5], alpha=1e-6, beta=1e6, gamma=g, black_ridges=True,
+                     mode="reflect").cpu().numpy().reshape(-1)[ok]
+        e = rg[ok] * np.float32(-1.0 / (2.0 * g * g))
+        assert _ulps(out, -np.expm1(e.astype(np.float64))).max() <= 1.0
+    kw = dict(sigmas=[1.5], alpha=1e-6, beta=1e6, gamma=1e-30, black_ridges=True)
+    out = frangi(x, **kw).cpu().numpy().reshape(-1)
+    assert (out[ok] == 1).all()  # exponents of -inf
+    x[(shape[0] // 2,) * len(shape)] = float("nan")
+    assert np.isnan(frangi(x, **kw).cpu().numpy()).any()
