@@ -1177,14 +1177,11 @@ __global__ __launch_bounds__(256) void k_frangi_from_eig(const W* __restrict__ e
                                                          double alpha_sq, double beta_sq,
                                                          const double* gamma_sq_dev) {
   const double gsq = *gamma_sq_dev;
-  const FrangiNegRecip nrc = frangi_neg_recip(alpha_sq, beta_sq, gsq);
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * 256) {
     if (NDIM == 3) {
-      // float: as the final pass computes the later sigmas
-      const W l1 = e0[i], l2 = e1[i], l3 = e2[i], rg = frangi_rg3<W>(l1, l2, l3);
-      out[i] = sizeof(W) == 4 ? frangi_v3r<W>(l1, l2, l3, rg, nrc)
-                              : frangi_v3<W>(l1, l2, l3, rg, alpha_sq, beta_sq, gsq);
+      const W l1 = e0[i], l2 = e1[i], l3 = e2[i];
+      out[i] = frangi_v3<W>(l1, l2, l3, frangi_rg3<W>(l1, l2, l3), alpha_sq, beta_sq, gsq);
     } else {
       const W l1 = e0[i], l2 = e1[i];
       out[i] = frangi_v2<W>(l1, l2, frangi_rg2<W>(l1, l2), beta_sq, gsq);

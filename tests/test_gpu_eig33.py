@@ -192,3 +192,19 @@ def test_vesselness_one_minus_exp(gpu, shape):
     assert (out[ok] == 1).all()  # exponents of -inf
     x[(shape[0] // 2,) * len(shape)] = float("nan")
     assert np.isnan(frangi(x, **kw).cpu().numpy()).any()
+
+
+@pytest.mark.parametrize("shape", [(48, 50, 52), (300, 310)])
+def test_first_sigma_in_double(gpu, shape):
+    """The first sigma's vesselness, once gamma is known from its maximum, is
+    computed in double and rounded once: half an ulp (and 2^-52 over the
+    exponent, which is above 1e-6 where it is looked at)."""
+    from cucim_amd.skimage.filters import frangi
+
+    x, rg, ok = _gamma_factor(shape)
+    out = frangi(x, sigmas=[1.5], alpha=1e-6, beta=1e6, gamma=None, black_ridges=True,
+                 mode="reflect").cpu().numpy().reshape(-1)
+    gsq = 2 * (np.sqrt(np.float64(rg.max())) / 2) ** 2
+    e = -rg.astype(np.float64) / gsq
+    ok &= e < -1e-6
+    assert _ulps(out[ok], -np.expm1(e[ok])).max() <= 0.501
