@@ -835,7 +835,9 @@ int hc_separable2d_slices(const hc_array* in, const hc_array* out, const hc_taps
       taps1->anchor >= taps1->K)
     return fail(HC_ERR_VALUE, "invalid origin");
   rc = launch_sep2d_reg(in, out, taps0, taps1, mode0, mode1, cval, (hipStream_t)stream);
-  if (rc == -1) return fail(HC_ERR_RESOURCE, "not a float32 stack with kernels of at most 33 taps");
+  if (rc == -1)
+    return fail(HC_ERR_RESOURCE,
+                "not a float32 stack with kernels of at most 33 taps, or too many slices");
   return rc;
 }
 

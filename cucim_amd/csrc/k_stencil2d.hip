@@ -147,6 +147,10 @@ int launch_sep2d_reg(const hc_array* in, const hc_array* out, const hc_taps* t0,
   a.mode1 = mode1;
   a.cval = (float)cval;
   if (slices == 0 || a.H == 0 || a.W == 0) return HC_OK;
+  if (d0) {  // more tiles than a grid holds: left to the line kernels
+    constexpr int64_t TX = reg_strip_outputs(kRegMaxK);
+    if ((a.W + TX - 1) / TX > 0x7fffffff / slices / ((a.H + 7) / 8)) return -1;
+  }
   if (K <= 3) return launch_reg_ty<3>(a, slices, t0, t1, st);
   if (K <= 5) return launch_reg_ty<5>(a, slices, t0, t1, st);
   if (K <= 7) return launch_reg_ty<7>(a, slices, t0, t1, st);

@@ -75,6 +75,17 @@ def test_argument_errors_return_before_launch():
         _lib.check(_lib.ERR_RESOURCE)
 
 
+def test_stacks_of_too_many_tiles_are_left_to_the_line_kernels():
+    """More slices than a grid holds work-groups: refused as a matter of
+    resources, which the filters answer with separate passes."""
+    lib = _lib.load_library()
+    t, keep = _lib.make_taps(np.ones(3), 1, False)
+    for shape in ((1 << 31, 1, 4), (1 << 28, 100, 1000), ((1 << 62) // 8, 1, 1)):
+        a, b = _arr(shape), _arr(shape)
+        assert lib.hc_separable2d_slices(ctypes.byref(a), ctypes.byref(b), ctypes.byref(t),
+                                         ctypes.byref(t), 0, 0, 0.0, None) == _lib.ERR_RESOURCE
+
+
 def test_no_unresolved_library_symbols():
     """Every symbol of the library's own namespace is defined inside it (an
     unresolved one only fails when the GPU process loads it)."""
