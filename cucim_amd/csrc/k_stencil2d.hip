@@ -56,7 +56,7 @@ __global__ __launch_bounds__(256) void k_sep2d_reg(Reg2dArgs a, const RegTaps<K>
   } else {
 #pragma unroll
     for (int j = 0; j < TY + K - 1; ++j) {
-      const int64_t yr = remap(ya + j, a.H, a.mode0);
+      const int64_t yr = remap_near(ya + j, a.H, a.mode0);
       v[j] = (yr >= 0 && xr >= 0) ? a.in[yr * a.W + xr] : a.cval;
     }
   }
@@ -200,7 +200,7 @@ __global__ __launch_bounds__(256) void k_axis_reg(const AxisRegArgs a, const Reg
   } else {
 #pragma unroll
     for (int j = 0; j < TY + K - 1; ++j) {
-      const int64_t yr = remap(ya + j, a.N, a.mode);
+      const int64_t yr = remap_near(ya + j, a.N, a.mode);
       v[j] = a.in[base + (yr >= 0 ? yr : 0) * a.inner];
       if (yr < 0) v[j] = a.cval;
     }

@@ -181,8 +181,9 @@ int hc_separable2d(const hc_array* in, const hc_array* out, const hc_taps* taps0
                    const hc_taps* taps1, int mode0, int mode1, double cval,
                    void* stream);
 /* the same over the last two axes of a C-contiguous float32 (slices, H, W)
- * array in one launch; HC_ERR_RESOURCE for other dtypes or kernels of more
- * than 33 taps */
+ * array in one launch; HC_ERR_RESOURCE for other dtypes, kernels of more
+ * than 33 taps, and more slices than one launch takes.  Two hc_correlate1d
+ * calls are faster for short slices and long kernels. */
 int hc_separable2d_slices(const hc_array* in, const hc_array* out, const hc_taps* taps0,
                           const hc_taps* taps1, int mode0, int mode1, double cval, void* stream);
 

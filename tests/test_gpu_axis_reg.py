@@ -60,6 +60,44 @@ def test_stack_gaussian_equals_passes(gpu, monkeypatch, shape, sigma, mode):
         assert torch.equal(got, b)
 
 
+# slices of the fused launch's two row counts (8 up to 2^22 elements, 16 above),
+# whole and ragged tiles, kernels longer than a slice, and stacks that the rule
+# leaves to the line kernels
+_STACKS = [((20, 448, 512), 13, True), ((33, 386, 413), 33, True), ((600, 100, 225), 9, True),
+           ((700, 24, 333), 25, True), ((3000, 40, 24), 5, True), ((4000, 32, 40), 33, True),
+           ((4000, 5, 129), 25, True), ((300, 64, 512), (5, 33), True),
+           ((4000, 4, 260), 13, False), ((1500, 7, 300), 33, False), ((200, 10, 400), 33, False),
+           ((2000, 18, 300), 33, False), ((300, 27, 512), (5, 33), False)]
+
+
+@pytest.mark.parametrize("shape,K,fused", _STACKS)
+@pytest.mark.parametrize("mode", ["reflect", "mirror", "nearest", "wrap", "constant"])
+def test_stack_rule(gpu, monkeypatch, shape, K, fused, mode):
+    """The fused launch gives the separate passes' bits whether the rule takes
+    it or not."""
+    from cucim_amd import _array
+    from cucim_amd import _lib as L
+    from cucim_amd.skimage._vendored import _ndimage_filters as F
+
+    x = _view(shape, 0, 3, special=True)
+    rng = np.random.default_rng(1)
+    K0, K1 = K if isinstance(K, tuple) else (K, K)
+    w = [None] + [rng.standard_normal(k).astype(np.float32) for k in (K0, K1)]
+    t = [F._get_taps(v, v.size // 2, np.float32) for v in w[1:]]
+    out = torch.empty_like(x)
+    m = F._util._mode_code(mode)
+    rc = L.lib().hc_separable2d_slices(_array.hc_array(x), _array.hc_array(out), t[0].struct,
+                                       t[1].struct, m, m, 0.5, _array.stream())
+    assert rc == L.OK
+    assert F._stack_pays(*shape, K0, K1, shape[2] % 4 == 0) == fused
+    a = F._run_1d_correlates(x, (0, 1, 2), w, None, mode, 0.5)
+    monkeypatch.setattr(F, "FUSED_2D", False)
+    b = F._run_1d_correlates(x, (0, 1, 2), w, None, mode, 0.5)
+    for got in (a, out):
+        assert torch.equal(got.isnan(), b.isnan())
+        assert torch.equal(got.view(torch.int32)[~b.isnan()], b.view(torch.int32)[~b.isnan()])
+
+
 @pytest.mark.parametrize("n", [1, 7, 8, 9, 2047, 100003])
 @pytest.mark.parametrize("off", [0, 1, 3])
 def test_unsigned_to_float(gpu, n, off):
