@@ -240,12 +240,18 @@ int launch_axis_reg(const hc_array* in, const hc_array* out, const hc_taps* t, i
   if (!is_c_contiguous(in) || !is_c_contiguous(out)) return -1;
   const Lines ln = lines_of(in, axis);
   // The LDS line kernel's wide loads need rows that are whole 16-byte words:
-  // with them it is the faster one (8192^2, 17 taps: 113 us); without them, or
-  // where a wave's columns would span many rows, or in small arrays (8 to 10 us
-  // either way), the other way round (3000 x 4001, 17 taps: 48 us against 27).
+  // with them it is the faster one (8192^2, 17 taps: 113 us).  Without them this
+  // one is (3000 x 4001, 17 taps: 27 us against 48), except where a wave's
+  // columns would span many rows (axis strides below 32), in small arrays (8 to
+  // 10 us either way) and with long kernels over few lines: a work-group takes
+  // 256 lines whether they are there or not, the line kernel 64 (2^20 x 33: 13
+  // taps 187 us against 201, 17 taps 232 / 206; 2^19 x 65: 25 taps 181 / 227, 33
+  // taps 234 / 249; 2^18 x 127, 33 taps 135 / 127).
   const bool wide = ln.inner % 4 == 0 &&
                     (((uintptr_t)in->data | (uintptr_t)out->data) & 15) == 0;
-  if (wide || ln.inner < 32 || numel(in) < (int64_t)1 << 20) return -1;
+  const int64_t few = t->K <= 13 ? 0 : t->K <= 25 ? 64 : 128;
+  if (wide || ln.inner < 32 || ln.outer * ln.inner <= few || numel(in) < (int64_t)1 << 20)
+    return -1;
   AxisRegArgs a;
   std::memset(&a, 0, sizeof(a));
   a.in = (const float*)in->data;
