@@ -1,7 +1,8 @@
-"""The register line kernel of strided axes, the fused filter over stacks and
-the vector conversions: bit for bit what the element-wise kernel and the
-separate passes give, at tile edges, odd strides, unaligned arrays and with
-non-finite values."""
+"""The line kernels of strided axes (the register kernel where its rule takes
+the array, else the LDS kernel), the fused filter over stacks and the vector
+conversions: bit for bit what the element-wise kernel and the separate passes
+give, at tile edges, odd strides, unaligned arrays and with non-finite
+values."""
 
 import numpy as np
 import pytest
@@ -39,6 +40,30 @@ def test_strided_axis_equals_gather(gpu, shape, axis, K, origin, mode):
     b = ndi.correlate1d(x, w, algorithm="elementwise", **kw)
     assert torch.equal(a.view(torch.int32)[~b.isnan()], b.view(torch.int32)[~b.isnan()])
     assert torch.equal(a.isnan(), b.isnan())
+
+
+# float32 arrays that the register kernel takes (an axis stride that is no whole
+# number of 16-byte words, at least 32; 2^20 elements or more): both of its
+# heights, ragged tiles and strips, lines shorter than the kernel, one line more
+# than a strip holds, and the fewest lines for each kernel length
+@pytest.mark.parametrize("shape,axis,K,origin", [
+    ((33, 387, 1413), 0, 13, 0), ((33, 387, 1413), 1, 33, 5), ((201, 387, 413), 0, 7, -1),
+    ((70, 257, 1031), 1, 25, 0), ((1025, 3, 517), 0, 17, 2), ((5, 700, 401), 0, 33, 0),
+    ((2, 3, 180001), 0, 13, 0), ((2, 3, 180001), 1, 18, -3), ((1, 1, 1 << 20 | 1), 0, 5, 0),
+    ((4099, 257), 0, 33, 0), ((32000, 33), 0, 13, 0), ((16200, 65), 0, 25, 0),
+    ((8130, 129), 0, 33, -8), ((4, 8000, 33), 1, 4, 0)])
+@pytest.mark.parametrize("mode", ["reflect", "mirror", "nearest", "wrap", "constant"])
+def test_register_kernel_equals_gather(gpu, shape, axis, K, origin, mode):
+    from cucim_amd.skimage._vendored import ndimage as ndi
+
+    assert np.prod(shape) >= 1 << 20
+    x = _view(shape, 0, K + axis, special=True)
+    w = np.random.default_rng(K).standard_normal(K).astype(np.float32)
+    kw = dict(axis=axis, mode=mode, cval=1.5, origin=origin)
+    a = ndi.correlate1d(x, w, **kw)
+    b = ndi.correlate1d(x, w, algorithm="elementwise", **kw)
+    assert torch.equal(a.isnan(), b.isnan())
+    assert torch.equal(a.view(torch.int32)[~b.isnan()], b.view(torch.int32)[~b.isnan()])
 
 
 @pytest.mark.parametrize("shape", [(1, 5, 9), (3, 33, 240), (4, 17, 515), (2, 1, 300)])
