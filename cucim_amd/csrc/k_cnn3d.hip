@@ -602,8 +602,11 @@ int launch_24x24(ConvArgs a, int64_t batch, hipStream_t st) {
 
 int conv_24x24(const ConvArgs& a, int64_t batch, hipStream_t st) {
   // Blocks of 8 planes read less halo and fewer LDS words per product; blocks
-  // of 4 planes are half the work and divide better over 256 CUs where there
-  // are few.
+  // of 4 are half the work and divide better over 256 CUs where there are few.
+  // By rounds of work-groups, one layer with 8 against 4 planes (us): 64 / 128
+  // (258^3) 652 / 681, 16 / 32 (162^3) 160 / 166, 1 / 2 (58^3) 14.9 / 16.4; 12 /
+  // 23 (146^3) 124.9 / 123.1, 6 / 11 (114^3) 64.7 / 62.1, 4 / 7 (98^3) 47.0 /
+  // 42.7, 1 / 1 (22^3) 12.9 / 8.7.
   ConvArgs b = a;
   int rc = conv_blocks(&b, batch, 8);
   if (rc != HC_OK) return rc;
@@ -611,7 +614,7 @@ int conv_24x24(const ConvArgs& a, int64_t batch, hipStream_t st) {
   rc = conv_blocks(&b, batch, 4);
   if (rc != HC_OK) return rc;
   const int64_t n4 = (b.nblocks + 255) / 256;
-  return 10 * n8 <= 6 * n4 ? launch_24x24<8>(a, batch, st) : launch_24x24<4>(a, batch, st);
+  return 25 * n8 <= 13 * n4 ? launch_24x24<8>(a, batch, st) : launch_24x24<4>(a, batch, st);
 }
 
 }  // namespace
