@@ -158,21 +158,21 @@ __device__ __forceinline__ void eig33(F aa, F bb, F cc, F dd, F ee, F ff, int de
   // cos((phi - pi) / 3) and cos((phi + pi) / 3)
   double x1_term, ct, st;
   if constexpr (sizeof(F) == 4) {
-    if (x1 < HUGE_VAL && fabs(x2) < HUGE_VAL) {
-      // cos(phi) = x2 / (2 x1^(3/2)), sin(phi) = sqrt(4 x1^3 - x2^2) / (2 x1^(3/2));
-      // the difference is taken before the scaling, as below: from cos(phi)
-      // rounded, it would be up to 1.7 times further off where two eigenvalues
-      // meet.  x1 of floats is 0 or at least 1e-91; with x1 = 0 the angle does
-      // not matter.
-      const double y = x1 > 1e-200 ? rsqrt_fast(x1) : 0.0;
-      x1_term = (2.0 / 3.0) * (x1 * y);
-      const double h = 0.5 * y * y * y;
-      const double arg = fmax(4 * x1 * x1 * x1 - x2 * x2, 0.0);
-      const double sp = arg > 0.0 ? arg * rsqrt_fast(arg) * h : 0.0;
-      third_angle(x2 * h, sp, ct, st);
-    } else {
-      // an infinite or NaN element: the angles that the arctangent below
-      // gives there (x2 = +-inf: 0 or pi; x2 finite: pi / 2; NaN: NaN)
+    // cos(phi) = x2 / (2 x1^(3/2)), sin(phi) = sqrt(4 x1^3 - x2^2) / (2 x1^(3/2));
+    // the difference is taken before the scaling, as below: from cos(phi)
+    // rounded, it would be up to 1.7 times further off where two eigenvalues
+    // meet.  x1 of floats is 0 or at least 1e-91; with x1 = 0 the angle does
+    // not matter.
+    const double y = x1 > 1e-200 ? rsqrt_fast(x1) : 0.0;
+    x1_term = (2.0 / 3.0) * (x1 * y);
+    const double h = 0.5 * y * y * y;
+    const double arg = fmax(4 * x1 * x1 * x1 - x2 * x2, 0.0);
+    const double sp = arg > 0.0 ? arg * rsqrt_fast(arg) * h : 0.0;
+    third_angle(x2 * h, sp, ct, st);
+    if (!(fabs(ct) < 2.0)) {
+      // x1 infinite, or x2 infinite or NaN, all of which end so: an infinite or
+      // NaN element, and the angles that the arctangent below gives there (x2 =
+      // +-inf: 0 or pi; x2 finite: pi / 2; NaN: NaN)
       const double phi = x2 != x2 ? x2 : fabs(x2) < HUGE_VAL ? M_PI / 2.0 : x2 > 0 ? 0.0 : M_PI;
       x1_term = x1 < HUGE_VAL ? (2.0 / 3.0) * sqrt(x1) : x1;
       sincos_small(phi * third, ct, st);
