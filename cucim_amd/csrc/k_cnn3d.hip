@@ -21,10 +21,11 @@
 //       order (k_pack_weights).
 //   k_pad_bf16        reflect / nearest / ... padding of a float32 volume into
 //                     the bfloat16 single-channel input of the first layer
-//   training kernels  (float32): GELU backward, input gradient (full
-//                     correlation with the transposed kernel), weight / bias
-//                     gradients (per-block partial sums, atomically added),
-//                     masked MSE gradient, Adam step, bf16 packing.
+//   training kernels  (float32): MSE gradient, Adam step, bf16 packing.  The
+//                     training step takes its gradients from k_cnn3d_bwd.hip;
+//                     the GELU backward, input gradient and weight / bias
+//                     gradients here (one work-item per sum) serve the C
+//                     entries for one patch of any channel counts.
 #include <algorithm>
 #include <cmath>
 #include <cstring>

@@ -12,8 +12,9 @@
 // One training step of eight 64^3 patches took 269 ms with one work-item per
 // output and one launch per patch (weight gradients 40 launches of 3.4 ms,
 // each with an atomic add per weight and work-group; input gradients 32 of
-// 4.1 ms); it takes 6.3 ms with these (24 -> 24 layers: three launches of
-// 0.82 ms and three of 0.89 ms for all patches).
+// 4.1 ms); it takes 5.8 ms with these (24 -> 24 layers: three launches of
+// 0.76 ms and three of 0.87 ms for all patches, the matrix cores busy for 71
+// and 63 % of them, on 24 of 32 rows or columns).
 #include <algorithm>
 #include <cstring>
 

@@ -175,8 +175,8 @@ def test_edge_magnitude_bit_exact(gpu, shape, mode, rows):
 
 
 def test_edge_magnitude_unaligned_and_knob(gpu):
-    """A view that starts 4 bytes into its buffer takes the per-element
-    strips; the rows knob accepts only its listed values."""
+    """A view that starts 4 bytes into its buffer (vector loads at element
+    alignment); the rows knob accepts only its listed values."""
     from cucim_amd import _lib
     from cucim_amd.skimage.filters import sobel
 
