@@ -48,6 +48,18 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
+// The vesselness of one sample, not inlined: the constants of its double
+// arithmetic would be kept in registers through the contractions' loops (106
+// registers instead of 64, 25.2 ms per check of a 512^3 volume instead of 20.1).
+__device__ __noinline__ float check_vesselness(float h0, float h1, float h2, float h3, float h4,
+                                               float h5, double alpha_sq, double beta_sq,
+                                               double gamma_sq) {
+  float l1, l2, l3;
+  // (H00, H01, H02, H11, H12, H22) -> (a, d, f, b, e, c)
+  eig33<float>(h0, h3, h5, h1, h4, h2, 0, 1, l1, l2, l3);
+  return frangi_v3<float>(l1, l2, l3, frangi_rg3<float>(l1, l2, l3), alpha_sq, beta_sq, gamma_sq);
+}
+
 __global__ __launch_bounds__(256) void k_frangi_check(const CheckArgs a) {
   __shared__ float Cx[4][kChkMaxL][3];
   __shared__ float Cy[kChkMaxZ][6];
@@ -124,11 +136,8 @@ __global__ __launch_bounds__(256) void k_frangi_check(const CheckArgs a) {
         for (int u = 0; u < L; ++u) h = fmaf(kz[u], Cy[tid + u][e], h);
         Hm[e] = a.sign * h;
       }
-      float l1, l2, l3;
-      // (H00, H01, H02, H11, H12, H22) -> (a, d, f, b, e, c)
-      eig33<float>(Hm[0], Hm[3], Hm[5], Hm[1], Hm[4], Hm[2], 0, 1, l1, l2, l3);
-      const float rg = frangi_rg3<float>(l1, l2, l3);
-      const float v = frangi_v3<float>(l1, l2, l3, rg, a.alpha_sq, a.beta_sq, a.gamma_sq);
+      const float v = check_vesselness(Hm[0], Hm[1], Hm[2], Hm[3], Hm[4], Hm[5], a.alpha_sq,
+                                       a.beta_sq, a.gamma_sq);
       res[tid] = s == 0 ? v : nanmax(res[tid], v);
     }
     __syncthreads();
